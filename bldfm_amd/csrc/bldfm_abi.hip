@@ -515,7 +515,9 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
       D.off_aw = D.off_q0 = -1;
     }
     D.off_z = off_ws; off_ws += (int64_t)D.nslot * D.nxb * D.nyb;
-    D.off_nyq = off_ws; off_ws += (int64_t)D.nslot * (D.nlx + D.nly) * 2;
+    D.nyq_direct = nyq_is_direct(D.nlx, D.nly, D.nxb, D.nyb);
+    D.off_nyq = off_ws;
+    if (!D.nyq_direct) off_ws += (int64_t)D.nslot * (D.nlx + D.nly) * 2;
     D.off_v = off_ws; off_ws += (int64_t)D.nslot * D.nxb * D.ny;
     if (xlayout == 2) { D.off_vt = off_ws; off_ws += (int64_t)D.nslot * D.nxb * D.ny; }
     D.off_out = off_out; off_out += (int64_t)D.nslot * D.ny * D.nx;
@@ -533,7 +535,7 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
     off_ws += long_elems;
 
     // tiles: tab, fwd_rows, fwd_cols, shoot, nyq, inv_cols, inv_rows
-    const int fixc = nyq_fix_count(D.nlx, D.nly, D.nxb, D.nyb);
+    const int fixc = D.nyq_direct ? 0 : nyq_fix_count(D.nlx, D.nly, D.nxb, D.nyb);
     const int64_t nspot = (D.lanes + BLDFM_SUR_SPOT_STRIDE - 1) / BLDFM_SUR_SPOT_STRIDE;
     // lines of each pass; a split axis moves them to the four-step tiles
     const int64_t lines_fr = D.footprint ? 0 : D.ny, lines_fc = D.footprint ? 0 : D.nlx;

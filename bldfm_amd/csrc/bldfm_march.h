@@ -36,18 +36,23 @@ __device__ __forceinline__ bool lane_setup(const cdesc_t& D, int lane, Lane& L) 
   return true;
 }
 
-// Packed output of one mode (after complex64 rounding and phase shift).
+// Packed output of one mode (after complex64 rounding and phase shift).  An
+// unpaired Nyquist mode whose mirror is no retained mode (D.nyq_direct: the
+// band has both +-nl/2) is half of its Hermitian part at k and half of its
+// conjugate at -k, so it is written like a pair, times 1/2 (this saves the
+// k_nyq_fix launch, 4.6 us of a lone solve); otherwise X is kept for it.
 __device__ __forceinline__ void emit_mode(const cdesc_t& D, const Lane& L, double2* __restrict__ ws,
                                           int s, double2 Xp, double2 Xq, double2 sh) {
   if (D.single) { Xp = round_c64(Xp); Xq = round_c64(Xq); }
   if (D.has_shift) { Xp = ncmul(Xp, sh); Xq = ncmul(Xq, sh); }
-  if (L.kind == LANE_HALF) {
+  if (L.kind == LANE_HALF || D.nyq_direct) {
     const int cx = compact_of_freq(L.fx, D.nxb), cy = compact_of_freq(L.fy, D.nyb);
     const int mx = compact_mirror(cx, D.nxb), my = compact_mirror(cy, D.nyb);
     double2* Z = ws + D.off_z + (int64_t)s * D.nxb * D.nyb;
+    const double f = L.kind == LANE_HALF ? 1.0 : 0.5;
     // Z(k) = Xp + i Xq ; Z(-k) = conj(Xp) + i conj(Xq)
-    Z[(int64_t)cx * D.nyb + cy] = cmk(Xp.x - Xq.y, Xp.y + Xq.x);
-    Z[(int64_t)mx * D.nyb + my] = cmk(Xp.x + Xq.y, Xq.x - Xp.y);
+    Z[(int64_t)cx * D.nyb + cy] = cmk(f * (Xp.x - Xq.y), f * (Xp.y + Xq.x));
+    Z[(int64_t)mx * D.nyb + my] = cmk(f * (Xp.x + Xq.y), f * (Xq.x - Xp.y));
   } else {  // LANE_NYQ: keep X for the Hermitian fix-up
     double2* N = ws + D.off_nyq + ((int64_t)s * (D.nlx + D.nly) + L.nidx) * 2;
     N[0] = Xp;
@@ -58,7 +63,13 @@ __device__ __forceinline__ void emit_mode(const cdesc_t& D, const Lane& L, doubl
 __device__ __forceinline__ void emit_origin(const cdesc_t& D, double2* __restrict__ ws, int s,
                                             double p00, double q00) {
   if (D.single) { p00 = (double)(float)p00; q00 = (double)(float)q00; }
-  ws[D.off_z + (int64_t)s * D.nxb * D.nyb] = cmk(p00, q00);
+  double2* Z = ws + D.off_z + (int64_t)s * D.nxb * D.nyb;
+  Z[0] = cmk(p00, q00);
+  if (D.nyq_direct && D.nxb > D.nlx && D.nyb > D.nly) {
+    // (+nlx/2, -nly/2) and its mirror: the two corners no mode reaches
+    Z[(int64_t)(D.nlx / 2) * D.nyb + compact_of_freq(-D.nly / 2, D.nyb)] = cmk(0.0, 0.0);
+    Z[(int64_t)compact_of_freq(-D.nlx / 2, D.nxb) * D.nyb + D.nly / 2] = cmk(0.0, 0.0);
+  }
 }
 
 // e^{i(lx*shx + ly*shy)} (src/bldfm/solver.py:254-262)

@@ -134,6 +134,7 @@ struct InstDesc {
   int64_t off_out;      // output element offset: (nslot, ny, nx)
   int64_t off_long;     // workspace double2: four-step scratch (lines x n of the longest split pass)
   int32_t long_x, long_y;  // 1: the padded x / y length is split (four-step passes)
+  int32_t nyq_direct;      // 1: every Nyquist mode's mirror is outside the retained modes
 };
 
 // ---------------------------------------------------------------- frequencies
@@ -168,6 +169,18 @@ BLDFM_HD int nyq_count(int nlx, int nly) {
   if (nly % 2 == 0) n += nlx;
   if (nlx % 2 == 0) n += 2 * paired_max(nly) + 1;
   return n;
+}
+
+// Whether no Nyquist mode has its mirror among the retained modes: each axis
+// has no Nyquist frequency (odd nl) or a band with both +nl/2 and -nl/2.
+BLDFM_HD int nyq_is_direct(int nlx, int nly, int nxb, int nyb) {
+  return (nlx % 2 || nxb > nlx) && (nly % 2 || nyb > nly);
+}
+
+// Lane of the (0,0) mode (see decode_lane).
+BLDFM_HD int origin_lane(int nlx, int nly) {
+  const int Px = paired_max(nlx), Py = paired_max(nly);
+  return Py * (2 * Px + 1) + Px;
 }
 
 // Shooting lanes: upper half plane + positive x axis + origin + Nyquist.

@@ -169,3 +169,15 @@ def test_bench_refuses_multi_gpu():
     res = subprocess.run([sys.executable, str(ROOT / "bench.py"), "--gpus", "2"], capture_output=True, text=True,
                          timeout=120)
     assert res.returncode == 2 and "one GPU" in res.stderr
+
+
+def test_nyquist_direct_emission(tmp_path):
+    """Compile tests/native/nyq_direct_check.cpp: shooting lanes that write
+    the Nyquist modes themselves cover the packed band exactly once, with the
+    values of the Hermitian fix-up."""
+    exe = tmp_path / "nyq_direct_check"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-ffp-contract=off", "-o", str(exe),
+                    str(ROOT / "tests" / "native" / "nyq_direct_check.cpp")], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
+    assert int(out.stdout.split()[2]) > 100, out.stdout
