@@ -5,8 +5,10 @@
 #include <string.h>
 
 #include <cmath>
+#include <complex>
 
 #include <algorithm>
+#include <array>
 #include <map>
 #include <mutex>
 #include <string>
@@ -99,6 +101,101 @@ void twiddles(int n, double2* w) {
     w[t].x = w[n - t].x;
     w[t].y = -w[n - t].y;
   }
+}
+
+// ----------------------------------------------------------- chirp transforms
+typedef std::complex<long double> cld;
+
+cld mul(const cld& x, const cld& y) {
+  return cld(x.real() * y.real() - x.imag() * y.imag(), x.real() * y.imag() + x.imag() * y.real());
+}
+
+// e^{-2 pi i t/M}, t < M, for the longest chirp length M (once per process).
+const cld* pow2_roots() {
+  static const std::vector<cld> w = [] {
+    const int M = 1 << LINE_MAX_LM;
+    std::vector<cld> r(M);
+    for (int t = 0; t < M; ++t) {
+      const long double x = 2.0L * acosl(-1.0L) * t / M;
+      r[t] = 4 * t % M ? cld(cosl(x), -sinl(x)) : cld((t == 0) - (2 * t == M), (4 * t == 3 * M) - (4 * t == M));
+    }
+    return r;
+  }();
+  return w.data();
+}
+
+// Tables of a chirp line (bldfm_line.h): A[u] = V^{(i0+u)^2},
+// B[v] = V^{(o0+v)^2} with V = e^{-i pi/N}, and H = DFT_M(h)/M of the circular
+// kernel h[d] = V^{-(o0-i0+d)^2}, -nin < d < nout.  Angles are reduced exactly
+// (squares modulo 2N) and everything is formed in extended precision.
+int line_table_len(const LineAlg& a) { return a.nin + a.nout + (1 << a.lm); }
+
+void line_tables(const LineAlg& a, double2* out) {
+  const int N2 = 2 * a.N, M = 1 << a.lm, step = 64;
+  const long double pi = acosl(-1.0L);
+  auto unit = [&](long double x) { return cld(cosl(x), -sinl(x)); };
+  // V^t from two short tables: 64 + 2N/64 evaluations instead of 2N
+  std::vector<cld> lo(step), hi(N2 / step + 1);
+  for (int t = 0; t < step; ++t) lo[t] = unit(pi * t / a.N);
+  for (int t = 0; t <= N2 / step; ++t) hi[t] = unit(pi * ((int64_t)t * step) / a.N);
+  auto V2 = [&](int64_t k) {  // V^{k^2}
+    const int t = (int)(k * k % N2);
+    return mul(hi[t / step], lo[t % step]);
+  };
+  auto put = [&](const cld& z) { out->x = (double)z.real(); out->y = (double)z.imag(); ++out; };
+  for (int u = 0; u < a.nin; ++u) put(V2(a.i0 + u));
+  for (int v = 0; v < a.nout; ++v) put(V2(a.o0 + v));
+  std::vector<cld> h(M, cld(0, 0));
+  std::vector<int> rev(M);
+  for (int i = 1; i < M; ++i) rev[i] = rev[i >> 1] >> 1 | (i & 1) << (a.lm - 1);
+  for (int d = 1 - a.nin; d < a.nout; ++d) {
+    const cld v = V2((int64_t)a.o0 - a.i0 + d);
+    h[rev[d & (M - 1)]] = cld(v.real() / M, -v.imag() / M);
+  }
+  const cld* w = pow2_roots();
+  for (int i = 0; i < M; i += 2) {
+    const cld p = h[i], q = h[i + 1];
+    h[i] = p + q;
+    h[i + 1] = p - q;
+  }
+  for (int len = 4; len <= M; len *= 2)
+    for (int i = 0; i < M; i += len)
+      for (int j = 0; j < len / 2; ++j) {
+        const cld p = h[i + j], q = mul(h[i + j + len / 2], w[j * ((1 << LINE_MAX_LM) / len)]);
+        h[i + j] = p + q;
+        h[i + j + len / 2] = p - q;
+      }
+  for (int i = 0; i < M; ++i) put(h[i]);
+}
+
+// How one pass of one instance runs: as a chirp where N has a prime factor
+// above 5 and the chirp's line is the cheaper one.  Both costs are fits of
+// measured passes (us per 1e6 lines, batches of 64^2 to 1000^2 footprints, y-pass):
+// the mixed-radix line of N points takes about N times its stages' sum below,
+// 0.76 p for a prime p > 5 that runs as p products a point, plus 450 (at least
+// 1650: a line is never less than one wave); the chirp takes 1262, 1536, 2836,
+// 7373 and 17760 at M = 128 ... 2048, where from 1024 on a line spans waves.
+// On lengths with factors 2, 3 and 5 alone the chirp is within +-20% of the
+// mixed-radix line up to M = 512 and slower above, so those keep the one
+// transform, whose error is the smaller (conc 3.9-7e-16 against 5-9e-16).
+LineAlg choose_line(int N, int nin, int i0, int nout, int o0) {
+  LineAlg a;
+  memset(&a, 0, sizeof(a));
+  a.N = N; a.nin = nin; a.i0 = i0; a.nout = nout; a.o0 = o0;
+  int lm = LINE_MIN_LM, rest = N;
+  while (lm <= LINE_MAX_LM && nin + nout - 1 > (1 << lm)) ++lm;
+  if (lm > LINE_MAX_LM) return a;
+  double stages = 0.0;
+  for (; rest % 8 == 0; rest /= 8) stages += 0.85;
+  for (; rest % 2 == 0; rest /= 2) stages += 0.4;
+  for (; rest % 3 == 0; rest /= 3) stages += 0.95;
+  for (; rest % 5 == 0; rest /= 5) stages += 1.15;
+  if (rest == 1) return a;
+  for (int p = 7; rest > 1; p += 2)
+    for (; rest % p == 0; rest /= p) stages += 0.76 * p;
+  const double chirp[] = {1250.0, 1262.0, 1536.0, 2836.0, 7373.0, 17760.0};
+  if (chirp[lm - LINE_MIN_LM] < std::max(1650.0, 450.0 + stages * N)) a.lm = lm;
+  return a;
 }
 
 int fft_threads_for(int n) {
@@ -230,6 +327,7 @@ struct bldfm_plan {
   std::vector<InstDesc> desc;
   void* dmeta = nullptr;  // device metadata blob
   PlanDev dev{};
+  LinePlan lines{};
   size_t ws_bytes = 0;
   int64_t tab_doubles = 0, ws_cplx = 0, prof_doubles = 0, src_doubles = 0, out_elems = 0;
   // phase timing (bldfm_plan_timing_begin/end): 7 events per execution
@@ -374,15 +472,19 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
   std::vector<int32_t> met_flag(ninst, 0);
   std::vector<int32_t> ints;
   std::vector<int> plan_n;  // distinct transform lengths
+  std::vector<int64_t> roots(LINE_NLM, -1);  // twiddle tables of the chirp lengths, behind the twiddles
+  std::vector<char> mixed;  // lengths that a mixed-radix line runs (the others need no twiddles)
   auto plan_id = [&](int n) {
     for (size_t i = 0; i < plan_n.size(); ++i)
       if (plan_n[i] == n) return (int)i;
     plan_n.push_back(n);
+    mixed.push_back(0);
     return (int)plan_n.size() - 1;
   };
   // tab, fwd_rows, fwd_cols, shoot, nyq, inv_cols, inv_rows, sur, spot, transpose,
-  // then the four-step steps A, B of fwd_rows, fwd_cols, inv_cols, inv_rows
-  constexpr int kKinds = 18;
+  // then the four-step steps A, B of fwd_rows, fwd_cols, inv_cols, inv_rows,
+  // then the chirp lines of those four passes, by length
+  constexpr int kKinds = 18 + 4 * LINE_NLM;
   std::vector<int64_t> tiles[kKinds];
   for (auto& v : tiles) v.assign(ninst + 1, 0);
   std::vector<SurMet> surmet(ninst);
@@ -390,7 +492,10 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
   int64_t off_prof = 0, off_tab = 0, off_src = 0, off_ws = 0, off_out = 0;
   const int32_t* lv = levels;
   int out_f32 = -1, any_disp = 0, variant_used[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
-  int max_n = 1;
+  int max_n = 1, line_lds[4][LINE_NLM] = {};
+  int64_t ltab_len = 0;  // chirp tables, behind the twiddles
+  std::map<std::array<int, 6>, int64_t> ltab_at;
+  std::vector<LineAlg> ltab;
 
   auto bad = [&](int code, const std::string& m) {
     if (P->dmeta) (void)hipFree(P->dmeta);
@@ -451,8 +556,8 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
     if (!D.footprint) any_disp = 1;
     D.plan_x = plan_id(Lx);
     D.plan_y = plan_id(Ly);
-    if (split_x) { plan_id(split_x); plan_id(Lx / split_x); }
-    if (split_y) { plan_id(split_y); plan_id(Ly / split_y); }
+    for (const int n : {split_x, split_x ? Lx / split_x : 0, split_y, split_y ? Ly / split_y : 0})
+      if (n) mixed[plan_id(n)] = 1;
     D.lanes = shoot_lanes(D.nlx, D.nly);
     D.dx = I.dx; D.dy = I.dy;
     if (!(I.dx > 0.0) || !(I.dy > 0.0)) return bad(BLDFM_EINVAL, "grid increments must be positive");
@@ -540,16 +645,45 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
     // lines of each pass; a split axis moves them to the four-step tiles
     const int64_t lines_fr = D.footprint ? 0 : D.ny, lines_fc = D.footprint ? 0 : D.nlx;
     const int64_t lines_ic = (int64_t)D.nslot * D.nxb, lines_ir = (int64_t)D.nslot * D.ny;
+    if (!D.long_x) {
+      const int bx = D.nxb - (D.nxb + 1) / 2, fx = D.nlx - (D.nlx + 1) / 2;
+      if (!D.footprint) D.line[0] = choose_line(Lx, D.nx, D.px, D.nlx, -fx);
+      D.line[3] = choose_line(Lx, D.nxb, -bx, D.nx, D.px);
+    }
+    if (!D.long_y) {
+      const int by = D.nyb - (D.nyb + 1) / 2, fy = D.nly - (D.nly + 1) / 2;
+      if (!D.footprint) D.line[1] = choose_line(Ly, D.ny, D.py, D.nly, -fy);
+      D.line[2] = choose_line(Ly, D.nyb, -by, D.ny, D.py);
+    }
+    if (!D.line[3].lm || (!D.footprint && !D.line[0].lm)) mixed[D.plan_x] = 1;
+    if (!D.line[2].lm || (!D.footprint && !D.line[1].lm)) mixed[D.plan_y] = 1;
+    for (int k = 0; k < 4; ++k) {
+      LineAlg& a = D.line[k];
+      if (!a.lm) continue;
+      if (roots[a.lm - LINE_MIN_LM] < 0) {
+        roots[a.lm - LINE_MIN_LM] = ltab_len;
+        ltab_len += 1 << a.lm;
+      }
+      int& lds = line_lds[k][a.lm - LINE_MIN_LM];
+      lds = std::max(lds, line_lds_bytes(a.lm, a.nin, k == PASS_FWD_COLS || k == PASS_INV_ROWS));
+      const std::array<int, 6> key = {a.N, a.i0, a.nin, a.o0, a.nout, a.lm};
+      auto at = ltab_at.emplace(key, ltab_len);
+      if (at.second) {
+        ltab.push_back(a);
+        ltab_len += line_table_len(a);
+      }
+      a.tab = at.first->second;
+    }
     const int64_t x1 = split_x, x2 = split_x ? Lx / split_x : 0;
     const int64_t y1 = split_y, y2 = split_y ? Ly / split_y : 0;
-    const int64_t nt[kKinds] = {
+    int64_t nt[kKinds] = {
         (D.nz + 255) / 256,
-        D.long_x ? 0 : lines_fr,
-        D.long_y ? 0 : lines_fc,
+        D.long_x || D.line[0].lm ? 0 : lines_fr,
+        D.long_y || D.line[1].lm ? 0 : lines_fc,
         (D.lanes + shoot_block - 1) / shoot_block,
         fixc > 0 ? (int64_t)D.nslot * ((fixc + 255) / 256) : 0,
-        D.long_y ? 0 : lines_ic,
-        D.long_x ? 0 : lines_ir,
+        D.long_y || D.line[2].lm ? 0 : lines_ic,
+        D.long_x || D.line[3].lm ? 0 : lines_ir,
         want_sur ? (D.lanes + SUR_PTS - 1) / SUR_PTS : 0,
         want_sur ? (nspot + 255) / 256 : 0,
         xlayout == 2 ? (int64_t)D.nslot * ((D.nxb + 31) / 32) * ((D.ny + 31) / 32) : 0,
@@ -557,7 +691,14 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
         lines_fr * x2, lines_fr * x1, lines_fc * y2, lines_fc * y1,
         lines_ic * y2, lines_ic * y1, lines_ir * x2, lines_ir * x1,
     };
-    for (int k = 10; k < kKinds; ++k)
+    const int64_t lines_of[4] = {lines_fr, lines_fc, lines_ic, D.ny};
+    for (int k = 0; k < 4; ++k) {  // chirp lines; the x-pass groups lines of one slot
+      const LineAlg& a = D.line[k];
+      if (!a.lm) continue;
+      const int64_t nl = line_per_wg(a.lm);
+      nt[18 + k * LINE_NLM + a.lm - LINE_MIN_LM] = (lines_of[k] + nl - 1) / nl * (k == 3 ? D.nslot : 1);
+    }
+    for (int k = 10; k < 18; ++k)
       if (nt[k] >= ((int64_t)1 << 31)) return bad(BLDFM_ELIMIT, "too many four-step transforms in one instance");
     for (int k = 0; k < kKinds; ++k) tiles[k][i + 1] = tiles[k][i] + nt[k];
   }
@@ -605,10 +746,26 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
       return bad(BLDFM_ELIMIT, "too many FFT stages");
     }
     plans[k].tw_off = tw_total;
-    tw_total += n;
+    if (mixed[k]) tw_total += n;
   }
-  std::vector<double2> tw(tw_total);
-  for (size_t k = 0; k < plan_n.size(); ++k) twiddles(plan_n[k], tw.data() + plans[k].tw_off);
+  for (auto& D : P->desc)
+    for (LineAlg& a : D.line) {
+      if (!a.lm) continue;
+      a.tw = roots[a.lm - LINE_MIN_LM] + tw_total;
+      a.tab += tw_total;
+    }
+  std::vector<double2> tw(tw_total + ltab_len);
+  for (size_t k = 0; k < plan_n.size(); ++k)
+    if (mixed[k]) twiddles(plan_n[k], tw.data() + plans[k].tw_off);
+  for (int m = 0; m < LINE_NLM; ++m)
+    for (int t = 0, M = 1 << (m + LINE_MIN_LM); roots[m] >= 0 && t < M; ++t) {
+      const cld w = pow2_roots()[t << (LINE_MAX_LM - LINE_MIN_LM - m)];
+      tw[tw_total + roots[m] + t].x = (double)w.real();
+      tw[tw_total + roots[m] + t].y = (double)w.imag();
+    }
+  for (const LineAlg& a : ltab)
+    line_tables(a, tw.data() + tw_total + ltab_at[{a.N, a.i0, a.nin, a.o0, a.nout, a.lm}]);
+  tw_total += ltab_len;
 
   // device metadata blob
   size_t off = 0;
@@ -667,6 +824,15 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
     V.t_long[k] = (const TileRec*)(base + o_tiles[10 + k]);
     V.tot_long[k] = tiles[10 + k][ninst];
   }
+  int line_max = 0;
+  for (int k = 0; k < 4; ++k)
+    for (int m = 0; m < LINE_NLM; ++m) {
+      P->lines.recs[k][m] = (const TileRec*)(base + o_tiles[18 + k * LINE_NLM + m]);
+      P->lines.tot[k][m] = tiles[18 + k * LINE_NLM + m][ninst];
+      P->lines.lds[k][m] = line_lds[k][m];
+      line_max = std::max(line_max, line_lds[k][m]);
+    }
+  if (line_max) bldfm_set_line_lds_attr(line_max);
   V.tot_tr = tiles[9][ninst];
   V.shoot_block = shoot_block;
   V.xlayout = xlayout;
@@ -802,7 +968,7 @@ int bldfm_plan_execute(bldfm_plan* P, double* prof, const double* src, void* con
   B.mode = sur ? (int32_t*)(B.ws + P->off_mode) : nullptr;
   hipEvent_t* ev = nullptr;
   if (P->timing_count < P->timing_max) ev = P->events.data() + (BLDFM_PHASES + 1) * (P->timing_count++);
-  const int rc = bldfm_launch_all(P->dev, B, kGridCap, stream, ev);
+  const int rc = bldfm_launch_all(P->dev, P->lines, B, kGridCap, stream, ev);
   if (rc == -1999) return fail(BLDFM_EHIP, "hipEventRecord failed");
   if (rc) return fail(BLDFM_EHIP, std::string("kernel launch failed: ") +
                                       hipGetErrorString((hipError_t)(-(rc + 1000))));

@@ -49,6 +49,15 @@ struct PlanDev {
   int64_t tot_sur, tot_spot;
 };
 
+// Lines of the chirp passes (bldfm_line.h) by PassId and length
+// 2^(LINE_MIN_LM + k): tile records (device), tiles, dynamic LDS.  Host only
+// (as part of PlanDev it would be an argument of every kernel).
+struct LinePlan {
+  const TileRec* recs[4][LINE_NLM];
+  int64_t tot[4][LINE_NLM];
+  int32_t lds[4][LINE_NLM];
+};
+
 struct ExecBufs {
   double* prof;        // 6*nz doubles per instance
   const double* src;   // surface flux (dispersion instances)
@@ -60,10 +69,38 @@ struct ExecBufs {
   int32_t* mode;       // ninst: 0 surrogate accepted, 1 FP64 solver; null: every instance solved
 };
 
+// Blocks of a grid-stride launch over `tiles` tiles.
+static inline unsigned grid_for(int64_t tiles, int cap) {
+  return (unsigned)(tiles < cap ? (tiles > 0 ? tiles : 1) : cap);
+}
+#define LAUNCH_CHECK()                       \
+  do {                                       \
+    hipError_t e_ = hipGetLastError();       \
+    if (e_ != hipSuccess) return -(int)e_ - 1000; \
+  } while (0)
+
+// The four transform passes.
+enum PassId { PASS_FWD_ROWS = 0, PASS_FWD_COLS = 1, PASS_INV_COLS = 2, PASS_INV_ROWS = 3 };
+// Chirp lines of one pass (all lengths of the plan), and the
+// dynamic LDS limit of their kernels; one translation unit per pass.
+int bldfm_launch_lines(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int pass, int grid_cap, hipStream_t stream);
+int bldfm_lines_pass0(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int grid_cap, hipStream_t stream, int lds_attr);
+int bldfm_lines_pass1(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int grid_cap, hipStream_t stream, int lds_attr);
+int bldfm_lines_pass2(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int grid_cap, hipStream_t stream, int lds_attr);
+int bldfm_lines_pass3(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int grid_cap, hipStream_t stream, int lds_attr);
+
+// Mixed-radix lines of one pass, single-workgroup and four-step, and the
+// dynamic LDS limits of the mixed-radix kernels.
+int bldfm_launch_pass(const PlanDev& P, const ExecBufs& B, int pass, int64_t tiles, int grid_cap, hipStream_t stream);
+int bldfm_launch_long(const PlanDev& P, const ExecBufs& B, int pass, int grid_cap, hipStream_t stream);
+void bldfm_pass_lds_attr(int bytes);
+void bldfm_long_lds_attr(int bytes);
+void bldfm_fft2_lds_attr(int bytes);
+
 // ev (optional): BLDFM_PHASES + 1 events recorded at the phase boundaries
 // [level table | forward transform | surrogate and gate | shooting | Nyquist fix-up | y-pass | x-pass]
 #define BLDFM_PHASES 7
-int bldfm_launch_all(const PlanDev& P, const ExecBufs& B, int grid_cap, hipStream_t stream,
+int bldfm_launch_all(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int grid_cap, hipStream_t stream,
                      hipEvent_t* ev = nullptr);
 // Surrogate inference over the lanes of accepted instances (packed spectrum).
 int bldfm_launch_sur_plan(const PlanDev& P, const ExecBufs& B, int grid_cap, hipStream_t stream);
@@ -108,6 +145,7 @@ int bldfm_launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_
                       const double2* in, double2* mid, double2* scr, double2* out, int32_t sign, double scale,
                       int threads, int lds_bytes, int grid_cap, hipStream_t stream);
 void bldfm_set_fft_lds_attr(int bytes);
+void bldfm_set_line_lds_attr(int bytes);
 int bldfm_launch_stability(const double* x, int64_t n, double* psi, double* phi, hipStream_t stream);
 int bldfm_launch_wind(const double* spd, const double* dir, int64_t n, double* u, double* v, hipStream_t stream);
 int bldfm_launch_math_probe(int op, const double* a, const double* b, int64_t n, double* out, hipStream_t stream);

@@ -16,18 +16,7 @@
 // Work of a batch of instances is laid out as tiles with per-kernel prefix
 // sums; every kernel is a grid-stride loop over its tiles.
 #include "bldfm_internal.h"
-#include "bldfm_fft.h"
 #include "bldfm_march.h"
-
-#define FFT_SMALL_E 8     // values per thread per stage, 256-thread FFT kernels (n <= 2048)
-
-// Workgroups are dispatched round-robin over the 8 XCDs (each with its own
-// L2).  This bijection of [0, n) gives every XCD a contiguous range of tiles,
-// so neighbouring tiles that share cache lines run behind the same L2.
-__device__ __forceinline__ int64_t xcd_swizzle(int64_t b, int64_t n) {
-  const int64_t q = n >> 3, r = n & 7, x = b & 7, i = b >> 3;
-  return x * q + (x < r ? x : r) + i;
-}
 
 // ---------------------------------------------------------------- level table
 // Entry i < nz-1 (step from z_i to z_{i+1}, coefficients of the LOWER level,
@@ -151,6 +140,7 @@ __device__ void origin_numeric(const cdesc_t& D, const double* __restrict__ tab,
       term = (q00 * T[9]) * T[11];
     }
     const int n = D.nz - i0 < 64 ? D.nz - i0 : 64;
+#pragma unroll 1
     for (int j = 0; j < n; ++j) {
       if (l == j) mine = p00;
       p00 = p00 - lane_value(term, j);
@@ -464,255 +454,6 @@ __global__ __launch_bounds__(256) void k_km01(const Km01Dev* __restrict__ P, dou
   out[D.off + c] = f;
 }
 
-// ---------------------------------------------------------------- FFT passes
-extern __shared__ double2 smem[];
-
-// Sources (first stage) and sinks (last stage) of the transforms.  A band of
-// nb compact values (truncated order: f >= 0 first, then f < 0) occupies
-// padded indices [0, lo) and [n - (nb - lo), n) with lo = (nb + 1)/2; the
-// gap between the two halves is zero.
-struct Band {
-  int lo, hi_start, nb;
-  __device__ __forceinline__ Band(int nb_, int n) : lo((nb_ + 1) / 2), hi_start(n - (nb_ - (nb_ + 1) / 2)), nb(nb_) {}
-  // compact index of padded index i, or -1 in the gap
-  __device__ __forceinline__ int compact(int i) const { return i < lo ? i : (i >= hi_start ? i - hi_start + lo : -1); }
-};
-
-// Compact band at element stride `stride` in global memory.
-struct BandIn {
-  const double2* __restrict__ src;
-  int64_t stride;
-  Band band;
-  __device__ __forceinline__ double2 operator()(int i) const {
-    const int c = band.compact(i);
-    return c < 0 ? cmk(0.0, 0.0) : src[(int64_t)c * stride];
-  }
-};
-
-// Band of the spectrum, scaled, to a compact array.
-struct BandOut {
-  double2* __restrict__ dst;
-  double fct;
-  Band band;
-  __device__ __forceinline__ void operator()(int o, double2 v) const {
-    const int c = band.compact(o);
-    if (c >= 0) dst[c] = cscale(fct, v);
-  }
-};
-
-// cnt values (element stride `stride`) placed at [off, off + cnt), zeros
-// elsewhere; real input when `re` is set.
-template <class T_>
-struct PadIn {
-  const T_* __restrict__ src;
-  int64_t stride;
-  int off, cnt;
-  __device__ __forceinline__ double2 operator()(int i) const {
-    const unsigned t = (unsigned)(i - off);
-    if (t >= (unsigned)cnt) return cmk(0.0, 0.0);
-    if constexpr (sizeof(T_) == sizeof(double)) return cmk(src[(int64_t)t * stride], 0.0);
-    else return src[(int64_t)t * stride];
-  }
-};
-
-// Outputs [off, off + cnt) to an array with element stride `stride`.
-struct CropOut {
-  double2* __restrict__ dst;
-  int64_t stride;
-  int off, cnt;
-  __device__ __forceinline__ void operator()(int o, double2 v) const {
-    const unsigned t = (unsigned)(o - off);
-    if (t < (unsigned)cnt) dst[(int64_t)t * stride] = v;
-  }
-};
-
-// Outputs [off, off + cnt) split into conc = cm * Re and flx = Im.
-template <class T_>
-struct SplitOut {
-  T_* __restrict__ conc;
-  T_* __restrict__ flx;
-  double cm;
-  int off, cnt;
-  __device__ __forceinline__ void operator()(int o, double2 v) const {
-    const unsigned t = (unsigned)(o - off);
-    if (t < (unsigned)cnt) {
-      conc[t] = (T_)(cm * v.x);
-      flx[t] = (T_)v.y;
-    }
-  }
-};
-
-// One transform of a tile loop; `reuse`: not the workgroup's first tile.
-template <int MAXE, class In, class Out>
-__device__ __forceinline__ void fft_dir(bool inv, const cplan_t& F, const double2* __restrict__ tw, int tid, int T,
-                                        In in, Out out, bool reuse) {
-  const bldfm_fft::Lds buf = bldfm_fft::lds_view(smem, F.n);
-  if (inv) bldfm_fft::lds_fft<MAXE, true>(buf, (const FftPlan*)&F, tw + F.tw_off, tid, T, in, out, reuse);
-  else bldfm_fft::lds_fft<MAXE, false>(buf, (const FftPlan*)&F, tw + F.tw_off, tid, T, in, out, reuse);
-}
-
-// The four passes, each as a factory of (plan, source, sink, direction) for
-// one line of one instance: the single-workgroup kernels below and the
-// four-step kernels (k_long) of split lengths run the same definitions.
-enum PassId { PASS_FWD_ROWS = 0, PASS_FWD_COLS = 1, PASS_INV_COLS = 2, PASS_INV_ROWS = 3 };
-
-// Forward, rows: one surface-flux row y placed at [px, px+nx) of nxe points,
-// e^{-i} DFT, scale 1/nxe (numpy norm="forward"), keep the nlx retained
-// columns in truncated order.
-template <class Fn>
-__device__ __forceinline__ void pass_fwd_rows(const PlanDev& P, const ExecBufs& B, const cdesc_t& D, int64_t line,
-                                              Fn&& fn) {
-  const cplan_t& F = *(const cplan_t*)(P.plans + D.plan_x);
-  const int y = (int)line;
-  fn(F, PadIn<double>{B.src + D.off_src + (int64_t)y * D.nx, 1, D.px, D.nx},
-     BandOut{B.ws + D.off_aw + (int64_t)y * D.nlx, 1.0 / (double)F.n, Band(D.nlx, F.n)}, false);
-}
-
-// Forward, columns: retained column jx over y placed at [py, py+ny) of nye
-// points, e^{-i} DFT, scale 1/nye, keep the nly retained rows -> q^0 (x-major).
-template <class Fn>
-__device__ __forceinline__ void pass_fwd_cols(const PlanDev& P, const ExecBufs& B, const cdesc_t& D, int64_t line,
-                                              Fn&& fn) {
-  const cplan_t& F = *(const cplan_t*)(P.plans + D.plan_y);
-  const int jx = (int)line;
-  fn(F, PadIn<double2>{B.ws + D.off_aw + jx, D.nlx, D.py, D.ny},
-     BandOut{B.ws + D.off_q0 + (int64_t)jx * D.nly, 1.0 / (double)F.n, Band(D.nly, F.n)}, false);
-}
-
-// Inverse, y-pass: band column cx of slot s (line s*nxb + cx; compact rows
-// scattered to their padded indices), unnormalised DFT (e^{-i} footprint,
-// e^{+i} dispersion), keep the cropped rows [py, py+ny).
-template <class Fn>
-__device__ __forceinline__ void pass_inv_cols(const PlanDev& P, const ExecBufs& B, const cdesc_t& D, int64_t line,
-                                              Fn&& fn) {
-  const cplan_t& F = *(const cplan_t*)(P.plans + D.plan_y);
-  const BandIn in{B.ws + D.off_z + line * D.nyb, 1, Band(D.nyb, F.n)};
-  // layout 1: column cx of slot s lands at v[s][y][cx]
-  const int64_t s = line / D.nxb, cx = line % D.nxb;
-  const CropOut out = P.xlayout == 1 ? CropOut{B.ws + D.off_v + s * D.ny * D.nxb + cx, D.nxb, D.py, D.ny}
-                                     : CropOut{B.ws + D.off_v + line * D.ny, 1, D.py, D.ny};
-  fn(F, in, out, !D.footprint);
-}
-
-// Inverse, x-pass: cropped row y of slot s (line s*ny + y) over the band
-// columns, DFT, keep [px, px+nx); conc = Re, flx = Im.  Instances served by
-// the surrogate carry no concentration spectrum (conc 0).
-template <class Fn>
-__device__ __forceinline__ void pass_inv_rows(const PlanDev& P, const ExecBufs& B, const cdesc_t& D, int inst,
-                                              int64_t line, Fn&& fn) {
-  const int s = (int)(line / D.ny), y = (int)(line % D.ny);
-  const cplan_t& F = *(const cplan_t*)(P.plans + D.plan_x);
-  const BandIn in = P.xlayout == 0
-                        ? BandIn{B.ws + D.off_v + (int64_t)s * D.nxb * D.ny + y, D.ny, Band(D.nxb, F.n)}
-                        : BandIn{B.ws + (P.xlayout == 1 ? D.off_v : D.off_vt) + ((int64_t)s * D.ny + y) * D.nxb,
-                                 1, Band(D.nxb, F.n)};
-  const int64_t o = D.off_out + line * D.nx;
-  const double cm = (B.mode && B.mode[inst] == 0) ? 0.0 : 1.0;
-  if (D.out_f32)
-    fn(F, in, SplitOut<float>{(float*)B.conc + o, (float*)B.flx + o, cm, D.px, D.nx}, !D.footprint);
-  else
-    fn(F, in, SplitOut<double>{(double*)B.conc + o, (double*)B.flx + o, cm, D.px, D.nx}, !D.footprint);
-}
-
-template <class Fn>
-__device__ __forceinline__ void run_pass(int pass, const PlanDev& P, const ExecBufs& B, const cdesc_t& D, int inst,
-                                         int64_t line, Fn&& fn) {
-  switch (pass) {
-    case PASS_FWD_ROWS: pass_fwd_rows(P, B, D, line, fn); break;
-    case PASS_FWD_COLS: pass_fwd_cols(P, B, D, line, fn); break;
-    case PASS_INV_COLS: pass_inv_cols(P, B, D, line, fn); break;
-    default: pass_inv_rows(P, B, D, inst, line, fn); break;
-  }
-}
-
-// Single-workgroup transforms of one pass, one line per tile (XCD-swizzled
-// so that each XCD works on a contiguous range of lines).
-template <int MAXE, int MAXT, int PASS>
-__global__ __launch_bounds__(MAXT) void k_pass(PlanDev P, ExecBufs B) {
-  const int T = blockDim.x, tid = threadIdx.x;
-  const TileRec* recs = PASS == PASS_FWD_ROWS   ? P.t_fwd_rows
-                        : PASS == PASS_FWD_COLS ? P.t_fwd_cols
-                        : PASS == PASS_INV_COLS ? P.t_inv_cols
-                                                : P.t_inv_rows;
-  const int64_t tot = PASS == PASS_FWD_ROWS   ? P.tot_fwd_rows
-                      : PASS == PASS_FWD_COLS ? P.tot_fwd_cols
-                      : PASS == PASS_INV_COLS ? P.tot_inv_cols
-                                              : P.tot_inv_rows;
-  for (int64_t b = blockIdx.x; b < tot; b += gridDim.x) {
-    const int64_t t = gridDim.x >= tot ? xcd_swizzle(b, tot) : b;
-    const TileRec tr = tile_rec(recs, t);
-    const cdesc_t& D = *(const cdesc_t*)(P.desc + tr.inst);
-    run_pass(PASS, P, B, D, tr.inst, tr.local, [&](const cplan_t& F, auto in, auto out, bool inv) {
-      fft_dir<MAXE>(inv, F, P.tw, tid, T, in, out, b != blockIdx.x);
-    });
-  }
-}
-
-// Four-step sources and sinks: step A reads the strided sub-sequence
-// in(j1 n2 + j2) and stores the twiddled length-n1 result at scr[j2 n1 + k1];
-// step B reads scr[j2 n1 + k1] over j2 and writes X[k1 + n1 k2] through the
-// pass's own sink.
-template <class In>
-struct SubIn {
-  In in;
-  int n2, j2;
-  __device__ __forceinline__ double2 operator()(int j1) const { return in(j1 * n2 + j2); }
-};
-struct TwiddleOut {
-  double2* __restrict__ dst;      // scr + j2 n1
-  const double2* __restrict__ w;  // W_n^t, t < n
-  int j2;
-  bool inv;
-  __device__ __forceinline__ void operator()(int k1, double2 v) const {
-    double2 t = w[j2 * k1];  // j2 k1 < n: no reduction modulo n
-    if (inv) t.y = -t.y;
-    dst[k1] = cmul(v, t);
-  }
-};
-struct ScrIn {
-  const double2* __restrict__ src;  // scr + k1
-  int n1;
-  __device__ __forceinline__ double2 operator()(int j2) const { return src[(int64_t)j2 * n1]; }
-};
-template <class Out>
-struct SubOut {
-  Out out;
-  int n1, k1;
-  __device__ __forceinline__ void operator()(int k2, double2 v) const { out(k1 + n1 * k2, v); }
-};
-
-// One step of the four-step transforms of the split lines of pass `pass`
-// (tile local = line * (n2 or n1) + sub-transform index).
-template <int MAXE, int MAXT, bool STEPB>
-__global__ __launch_bounds__(MAXT) void k_long(PlanDev P, ExecBufs B, int pass) {
-  const int T = blockDim.x, tid = threadIdx.x;
-  const int k = 2 * pass + (STEPB ? 1 : 0);
-  const TileRec* recs = P.t_long[k];
-  const int64_t tot = P.tot_long[k];
-  for (int64_t b = blockIdx.x; b < tot; b += gridDim.x) {
-    const TileRec tr = tile_rec(recs, b);
-    const cdesc_t& D = *(const cdesc_t*)(P.desc + tr.inst);
-    const bool x_axis = pass == PASS_FWD_ROWS || pass == PASS_INV_ROWS;
-    const cplan_t& FL = *(const cplan_t*)(P.plans + (x_axis ? D.plan_x : D.plan_y));
-    const int n = FL.n, n1 = FL.n1, n2 = FL.n2;
-    const int64_t per = STEPB ? n1 : n2;
-    const int64_t line = (int64_t)tr.local / per;
-    const int sub = (int)((int64_t)tr.local % per);
-    double2* scr = B.ws + D.off_long + line * n;
-    const bool reuse = b != blockIdx.x;
-    run_pass(pass, P, B, D, tr.inst, line, [&](const cplan_t&, auto in, auto out, bool inv) {
-      if constexpr (!STEPB) {
-        const cplan_t& F1 = *(const cplan_t*)(P.plans + FL.plan1);
-        fft_dir<MAXE>(inv, F1, P.tw, tid, T, SubIn<decltype(in)>{in, n2, sub},
-                      TwiddleOut{scr + (int64_t)sub * n1, P.tw + FL.tw_off, sub, inv}, reuse);
-      } else {
-        const cplan_t& F2 = *(const cplan_t*)(P.plans + FL.plan2);
-        fft_dir<MAXE>(inv, F2, P.tw, tid, T, ScrIn{scr + sub, n1}, SubOut<decltype(out)>{out, n1, sub}, reuse);
-      }
-    });
-  }
-}
-
 // x-pass layout 2: v[s][cx][y] -> vt[s][y][cx] in 32 x 32 tiles through LDS.
 // Reads run along y and writes along cx, both coalesced; the padding column
 // makes the transposed LDS reads (stride 33 x 16 bytes) conflict free.
@@ -743,17 +484,16 @@ __global__ __launch_bounds__(256) void k_transpose_v(PlanDev P, ExecBufs B) {
 }
 
 // ---------------------------------------------------------------- launcher
-static inline unsigned grid_for(int64_t tiles, int cap) {
-  return (unsigned)(tiles < cap ? (tiles > 0 ? tiles : 1) : cap);
+int bldfm_launch_lines(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int pass, int grid_cap, hipStream_t stream) {
+  switch (pass) {
+    case PASS_FWD_ROWS: return bldfm_lines_pass0(P, L, B, grid_cap, stream, 0);
+    case PASS_FWD_COLS: return bldfm_lines_pass1(P, L, B, grid_cap, stream, 0);
+    case PASS_INV_COLS: return bldfm_lines_pass2(P, L, B, grid_cap, stream, 0);
+    default: return bldfm_lines_pass3(P, L, B, grid_cap, stream, 0);
+  }
 }
 
-#define LAUNCH_CHECK()                       \
-  do {                                       \
-    hipError_t e_ = hipGetLastError();       \
-    if (e_ != hipSuccess) return -(int)e_ - 1000; \
-  } while (0)
-
-int bldfm_launch_all(const PlanDev& P, const ExecBufs& B, int grid_cap, hipStream_t stream,
+int bldfm_launch_all(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int grid_cap, hipStream_t stream,
                      hipEvent_t* ev) {
 #define MARK(k)                                            \
   if (ev) {                                                \
@@ -765,27 +505,13 @@ int bldfm_launch_all(const PlanDev& P, const ExecBufs& B, int grid_cap, hipStrea
     LAUNCH_CHECK();
   }
   MARK(1)
-  const unsigned ft = (unsigned)P.fft_threads;
-  const size_t lds = (size_t)P.fft_lds_bytes;
-  // single-workgroup lines of a pass, then its split (four-step) lines
-#define FFT_LAUNCH(PASS, tiles)                                                                        \
-  if ((tiles) > 0) {                                                                                   \
-    if (P.fft_small) k_pass<FFT_SMALL_E, 256, PASS><<<grid_for(tiles, grid_cap), ft, lds, stream>>>(P, B); \
-    else k_pass<BLDFM_FFT_MAXE, 1024, PASS><<<grid_for(tiles, grid_cap), ft, lds, stream>>>(P, B);        \
-    LAUNCH_CHECK();                                                                                    \
-  }                                                                                                    \
-  for (int st_ = 0; st_ < 2; ++st_) {                                                                  \
-    const int64_t tl_ = P.tot_long[2 * (PASS) + st_];                                                  \
-    if (tl_ <= 0) continue;                                                                            \
-    const unsigned g_ = grid_for(tl_, grid_cap);                                                       \
-    if (P.fft_small) {                                                                                 \
-      if (st_) k_long<FFT_SMALL_E, 256, true><<<g_, ft, lds, stream>>>(P, B, PASS);                    \
-      else k_long<FFT_SMALL_E, 256, false><<<g_, ft, lds, stream>>>(P, B, PASS);                       \
-    } else {                                                                                           \
-      if (st_) k_long<BLDFM_FFT_MAXE, 1024, true><<<g_, ft, lds, stream>>>(P, B, PASS);                \
-      else k_long<BLDFM_FFT_MAXE, 1024, false><<<g_, ft, lds, stream>>>(P, B, PASS);                   \
-    }                                                                                                  \
-    LAUNCH_CHECK();                                                                                    \
+  // chirp lines of a pass, then single-workgroup lines, then split (four-step) lines
+#define FFT_LAUNCH(PASS, tiles)                                                     \
+  {                                                                                 \
+    int rc_ = bldfm_launch_lines(P, L, B, PASS, grid_cap, stream);                  \
+    if (!rc_ && (tiles) > 0) rc_ = bldfm_launch_pass(P, B, PASS, tiles, grid_cap, stream); \
+    if (!rc_) rc_ = bldfm_launch_long(P, B, PASS, grid_cap, stream);                \
+    if (rc_) return rc_;                                                            \
   }
   if (P.any_dispersion) {
     FFT_LAUNCH(PASS_FWD_ROWS, P.tot_fwd_rows)
@@ -866,156 +592,21 @@ int bldfm_launch_profiles(const ProfSetup& S, double* out, hipStream_t stream) {
   return 0;
 }
 
-// ---------------------------------------------------------------- plain 2-D FFT
-// numpy fft2/ifft2 on `batch` contiguous (n0, n1) complex arrays: x-pass
-// over the rows into the workspace, then y-pass over the columns, output
-// multiplied by `scale`.
-struct StridedIn {
-  const double2* __restrict__ src;
-  int64_t stride;
-  __device__ __forceinline__ double2 operator()(int i) const { return src[(int64_t)i * stride]; }
-};
-struct StridedOut {
-  double2* __restrict__ dst;
-  int64_t stride;
-  double scale;
-  __device__ __forceinline__ void operator()(int o, double2 v) const { dst[(int64_t)o * stride] = cscale(scale, v); }
-};
-
-template <int MAXE>
-__device__ __forceinline__ void fft_plain(bool inv, const FftPlan* F, int n, const double2* __restrict__ tw, int tid,
-                                          int T, StridedIn in, StridedOut out, bool reuse) {
-  const bldfm_fft::Lds buf = bldfm_fft::lds_view(smem, n);
-  if (inv) bldfm_fft::lds_fft<MAXE, true>(buf, F, tw, tid, T, in, out, reuse);
-  else bldfm_fft::lds_fft<MAXE, false>(buf, F, tw, tid, T, in, out, reuse);
-}
-
-template <int MAXE, int MAXT>
-__global__ __launch_bounds__(MAXT) void k_fft2_rows(const FftPlan* F, const double2* __restrict__ tw,
-                                                  const double2* __restrict__ in, double2* __restrict__ mid,
-                                                  int32_t n, int64_t nrows, bool inv) {
-  const int T = blockDim.x, tid = threadIdx.x;
-  for (int64_t r = blockIdx.x; r < nrows; r += gridDim.x)
-    fft_plain<MAXE>(inv, F, n, tw, tid, T, StridedIn{in + r * n, 1}, StridedOut{mid + r * n, 1, 1.0},
-                    r != blockIdx.x);
-}
-
-template <int MAXE, int MAXT>
-__global__ __launch_bounds__(MAXT) void k_fft2_cols(const FftPlan* F, const double2* __restrict__ tw,
-                                                  const double2* __restrict__ mid, double2* __restrict__ out,
-                                                  int32_t n0, int32_t n1, int64_t ncols, double scale, bool inv) {
-  const int T = blockDim.x, tid = threadIdx.x;
-  for (int64_t w = blockIdx.x; w < ncols; w += gridDim.x) {
-    // eight neighbouring columns share every 128-byte line: each XCD takes a
-    // contiguous range of them, so a line is fetched into one L2 and not into
-    // eight (both passes of 2 x 2048^2 complex128: 302 -> 212 us)
-    const int64_t c = gridDim.x >= ncols ? xcd_swizzle(w, ncols) : w;
-    const int64_t b = c / n1, col = c % n1;
-    const int64_t o = b * (int64_t)n0 * n1 + col;
-    fft_plain<MAXE>(inv, F, n0, tw, tid, T, StridedIn{mid + o, n1}, StridedOut{out + o, n1, scale},
-                    w != blockIdx.x);
-  }
-}
-
-// Split (four-step) lines of the plain 2-D FFT: `rows` selects the rows of
-// the (n0, n1) arrays (line r at r*n1, stride 1), else their columns (line c
-// at (c / n1)*n0*n1 + c % n1, stride n1); scr holds nlines x n values.
-template <int MAXE, int MAXT, bool STEPB>
-__global__ __launch_bounds__(MAXT) void k_fft2_long(FftSplit S, const double2* __restrict__ in,
-                                                  double2* __restrict__ out, double2* __restrict__ scr, int rows,
-                                                  int32_t n0, int32_t n1, int64_t nlines, double scale, bool inv) {
-  const int T = blockDim.x, tid = threadIdx.x;
-  const int n = S.F->n, s1 = S.F->n1, s2 = S.F->n2;
-  const int64_t per = STEPB ? s1 : s2;
-  for (int64_t b = blockIdx.x; b < nlines * per; b += gridDim.x) {
-    const int64_t line = b / per;
-    const int sub = (int)(b % per);
-    const int64_t base = rows ? line * n1 : (line / n1) * (int64_t)n0 * n1 + line % n1;
-    const int64_t stride = rows ? 1 : n1;
-    double2* sc = scr + line * n;
-    const bldfm_fft::Lds buf0 = bldfm_fft::lds_view(smem, STEPB ? s2 : s1);
-    if constexpr (!STEPB) {
-      const SubIn<StridedIn> src{StridedIn{in + base, stride}, s2, sub};
-      const TwiddleOut dst{sc + (int64_t)sub * s1, S.tw, sub, inv};
-      if (inv) bldfm_fft::lds_fft<MAXE, true>(buf0, S.F1, S.tw1, tid, T, src, dst, b != blockIdx.x);
-      else bldfm_fft::lds_fft<MAXE, false>(buf0, S.F1, S.tw1, tid, T, src, dst, b != blockIdx.x);
-    } else {
-      const ScrIn src{sc + sub, s1};
-      const SubOut<StridedOut> dst{StridedOut{out + base, stride, scale}, s1, sub};
-      if (inv) bldfm_fft::lds_fft<MAXE, true>(buf0, S.F2, S.tw2, tid, T, src, dst, b != blockIdx.x);
-      else bldfm_fft::lds_fft<MAXE, false>(buf0, S.F2, S.tw2, tid, T, src, dst, b != blockIdx.x);
-    }
-  }
-}
-
-int bldfm_launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, int32_t batch,
-                      const double2* in, double2* mid, double2* scr, double2* out, int32_t sign, double scale,
-                      int threads, int lds_bytes, int grid_cap, hipStream_t stream) {
-  const bool inv = sign > 0;
-  const int64_t nrows = (int64_t)batch * n0, ncols = (int64_t)batch * n1;
-  // kernel family by the longest LDS transform (a split axis runs its two
-  // factors): the 256-thread kernels hold 8 values per thread, so they take
-  // lengths up to BLDFM_FFT_SMALL_N; a longer transform may still run on 256
-  // threads (10 values each) in the other family
-  auto lds_n = [](const FftSplit& A, int32_t n) { return A.F1 ? (A.n1 > A.n2 ? A.n1 : A.n2) : n; };
-  const int nmax = lds_n(A0, n0) > lds_n(A1, n1) ? lds_n(A0, n0) : lds_n(A1, n1);
-  const bool small = nmax <= BLDFM_FFT_SMALL_N;
-  if ((small && threads > 256) || threads > 1024 ||
-      (int64_t)threads * (small ? FFT_SMALL_E : BLDFM_FFT_MAXE) < nmax)
-    return -1000 - (int)hipErrorInvalidConfiguration;
-  // rows (axis 1, length n1): in -> mid
-  if (A1.F1) {
-    const unsigned ga = grid_for(nrows * A1.n2, grid_cap), gb = grid_for(nrows * A1.n1, grid_cap);
-    if (small) {
-      k_fft2_long<FFT_SMALL_E, 256, false><<<ga, threads, lds_bytes, stream>>>(A1, in, nullptr, scr, 1, n0, n1, nrows, 1.0, inv);
-      LAUNCH_CHECK();
-      k_fft2_long<FFT_SMALL_E, 256, true><<<gb, threads, lds_bytes, stream>>>(A1, nullptr, mid, scr, 1, n0, n1, nrows, 1.0, inv);
-    } else {
-      k_fft2_long<BLDFM_FFT_MAXE, 1024, false><<<ga, threads, lds_bytes, stream>>>(A1, in, nullptr, scr, 1, n0, n1, nrows, 1.0, inv);
-      LAUNCH_CHECK();
-      k_fft2_long<BLDFM_FFT_MAXE, 1024, true><<<gb, threads, lds_bytes, stream>>>(A1, nullptr, mid, scr, 1, n0, n1, nrows, 1.0, inv);
-    }
-  } else if (small) {
-    k_fft2_rows<FFT_SMALL_E, 256><<<grid_for(nrows, grid_cap), threads, lds_bytes, stream>>>(A1.F, A1.tw, in, mid, n1, nrows, inv);
-  } else {
-    k_fft2_rows<BLDFM_FFT_MAXE, 1024><<<grid_for(nrows, grid_cap), threads, lds_bytes, stream>>>(A1.F, A1.tw, in, mid, n1, nrows, inv);
-  }
-  LAUNCH_CHECK();
-  // columns (axis 0, length n0): mid -> out, scaled
-  if (A0.F1) {
-    const unsigned ga = grid_for(ncols * A0.n2, grid_cap), gb = grid_for(ncols * A0.n1, grid_cap);
-    if (small) {
-      k_fft2_long<FFT_SMALL_E, 256, false><<<ga, threads, lds_bytes, stream>>>(A0, mid, nullptr, scr, 0, n0, n1, ncols, 1.0, inv);
-      LAUNCH_CHECK();
-      k_fft2_long<FFT_SMALL_E, 256, true><<<gb, threads, lds_bytes, stream>>>(A0, nullptr, out, scr, 0, n0, n1, ncols, scale, inv);
-    } else {
-      k_fft2_long<BLDFM_FFT_MAXE, 1024, false><<<ga, threads, lds_bytes, stream>>>(A0, mid, nullptr, scr, 0, n0, n1, ncols, 1.0, inv);
-      LAUNCH_CHECK();
-      k_fft2_long<BLDFM_FFT_MAXE, 1024, true><<<gb, threads, lds_bytes, stream>>>(A0, nullptr, out, scr, 0, n0, n1, ncols, scale, inv);
-    }
-  } else if (small) {
-    k_fft2_cols<FFT_SMALL_E, 256><<<grid_for(ncols, grid_cap), threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
-  } else {
-    k_fft2_cols<BLDFM_FFT_MAXE, 1024><<<grid_for(ncols, grid_cap), threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
-  }
-  LAUNCH_CHECK();
-  return 0;
-}
-
 // Allow dynamic LDS beyond the default per-workgroup cap for the FFT kernels.
+void bldfm_set_line_lds_attr(int bytes) {
+  const PlanDev P{};
+  const LinePlan L{};
+  const ExecBufs B{};
+  (void)bldfm_lines_pass0(P, L, B, 0, nullptr, bytes);
+  (void)bldfm_lines_pass1(P, L, B, 0, nullptr, bytes);
+  (void)bldfm_lines_pass2(P, L, B, 0, nullptr, bytes);
+  (void)bldfm_lines_pass3(P, L, B, 0, nullptr, bytes);
+}
+
 void bldfm_set_fft_lds_attr(int bytes) {
-  const void* fns[] = {
-      (const void*)k_pass<FFT_SMALL_E, 256, PASS_FWD_ROWS>, (const void*)k_pass<FFT_SMALL_E, 256, PASS_FWD_COLS>,
-      (const void*)k_pass<FFT_SMALL_E, 256, PASS_INV_COLS>, (const void*)k_pass<FFT_SMALL_E, 256, PASS_INV_ROWS>,
-      (const void*)k_long<FFT_SMALL_E, 256, false>, (const void*)k_long<FFT_SMALL_E, 256, true>,
-      (const void*)k_fft2_rows<FFT_SMALL_E, 256>, (const void*)k_fft2_cols<FFT_SMALL_E, 256>,
-      (const void*)k_fft2_long<FFT_SMALL_E, 256, false>, (const void*)k_fft2_long<FFT_SMALL_E, 256, true>,
-      (const void*)k_pass<BLDFM_FFT_MAXE, 1024, PASS_FWD_ROWS>, (const void*)k_pass<BLDFM_FFT_MAXE, 1024, PASS_FWD_COLS>,
-      (const void*)k_pass<BLDFM_FFT_MAXE, 1024, PASS_INV_COLS>, (const void*)k_pass<BLDFM_FFT_MAXE, 1024, PASS_INV_ROWS>,
-      (const void*)k_long<BLDFM_FFT_MAXE, 1024, false>, (const void*)k_long<BLDFM_FFT_MAXE, 1024, true>,
-      (const void*)k_fft2_rows<BLDFM_FFT_MAXE, 1024>, (const void*)k_fft2_cols<BLDFM_FFT_MAXE, 1024>,
-      (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, false>, (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, true>};
-  for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  bldfm_pass_lds_attr(bytes);
+  bldfm_long_lds_attr(bytes);
+  bldfm_fft2_lds_attr(bytes);
 }
 
 // ---------------------------------------------------------------- elementwise

@@ -19,6 +19,14 @@ __device__ __forceinline__ TileRec tile_rec(const TileRec* recs, int64_t t) {
   return o;
 }
 
+// Workgroups are dispatched round-robin over the 8 XCDs (each with its own
+// L2).  This bijection of [0, n) gives every XCD a contiguous range of tiles,
+// so neighbouring tiles that share cache lines run behind the same L2.
+__device__ __forceinline__ int64_t xcd_swizzle(int64_t b, int64_t n) {
+  const int64_t q = n >> 3, r = n & 7, x = b & 7, i = b >> 3;
+  return x * q + (x < r ? x : r) + i;
+}
+
 // ---------------------------------------------------------------- shooting
 struct Lane {
   int kind, fx, fy, nidx;

@@ -78,6 +78,35 @@ BLDFM_HD int tw_table_len(int n) {
 // Dynamic LDS of one transform: buffer and twiddle tables.
 BLDFM_HD int fft_lds_bytes(int n) { return (n + tw_table_len(n)) * 16; }
 
+// Chirp transform of one pass of one instance on a power-of-two length
+// M = 2^lm (bldfm_line.h); lm = 0: the mixed-radix passes run the line.
+struct LineAlg {
+  int32_t lm, N;           // transform length N
+  int32_t nin, i0;         // input window: indices i0 .. i0 + nin - 1 (i0 may be negative)
+  int32_t nout, o0;        // output window
+  int64_t tw;              // twiddle table W_M^t (M entries)
+  int64_t tab;             // chirp tables A (nin), B (nout), H (M)
+};
+#define LINE_MIN_LM 6
+#define LINE_MAX_LM 11
+#define LINE_NLM (LINE_MAX_LM - LINE_MIN_LM + 1)
+
+// Lines per 256-thread workgroup, stage twiddles in LDS, pitch of the staged
+// lines (the lanes of an LDS access that go to different lines hit different
+// banks) and dynamic LDS of a tile, all for M = 2^lm.
+BLDFM_HD int line_per_wg(int lm) { return 2048 >> lm; }
+BLDFM_HD int line_tw_len(int lm) {
+  return lm == 6 ? 56 : lm == 7 ? 120 : lm == 8 ? 248 : lm == 9 ? 504 : lm == 10 ? 1016 : 2040;
+}
+BLDFM_HD int line_pitch(int lm, int nin) {
+  const int nl = line_per_wg(lm);
+  return (nin + 7) / 8 * 8 + (nl >= 8 ? 1 : nl == 1 ? 0 : 8 / nl);
+}
+BLDFM_HD int line_lds_bytes(int lm, int nin, bool staged) {
+  const int stage = staged ? line_per_wg(lm) * line_pitch(lm, nin) : 0;
+  return (line_tw_len(lm) + (stage > 2048 ? stage : 2048)) * 16;
+}
+
 // One tile of a kernel's work: the instance and the tile's index inside it.
 struct TileRec {
   int32_t inst;
@@ -134,6 +163,7 @@ struct InstDesc {
   int64_t off_out;      // output element offset: (nslot, ny, nx)
   int64_t off_long;     // workspace double2: four-step scratch (lines x n of the longest split pass)
   int32_t long_x, long_y;  // 1: the padded x / y length is split (four-step passes)
+  LineAlg line[4];         // forward rows, forward columns, inverse y-pass, inverse x-pass
   int32_t nyq_direct;      // 1: every Nyquist mode's mirror is outside the retained modes
 };
 
