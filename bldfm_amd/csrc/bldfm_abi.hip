@@ -599,7 +599,7 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
     D.max_level = max_level;
     D.variant = D.analytic ? 3 : (nfilled <= 1 ? 0 : (nfilled <= 4 ? 1 : 2));
     D.exact = I.fast ? 0 : 1;
-    variant_used[D.variant][D.exact] = 1;
+    D.plane = pair_lanes(D.nlx, D.nly);
     const bool want_sur = I.surrogate != 0 && I.prof_from_met && D.footprint;
     if (want_sur) {
       surmet[i] = sur_met_of(met[i], I.met.n);
@@ -680,7 +680,7 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
         (D.nz + 255) / 256,
         D.long_x || D.line[0].lm ? 0 : lines_fr,
         D.long_y || D.line[1].lm ? 0 : lines_fc,
-        (D.lanes + shoot_block - 1) / shoot_block,
+        0,  // shooting: below, once the plan's lanes are known
         fixc > 0 ? (int64_t)D.nslot * ((fixc + 255) / 256) : 0,
         D.long_y || D.line[2].lm ? 0 : lines_ic,
         D.long_x || D.line[3].lm ? 0 : lines_ir,
@@ -701,6 +701,25 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
     for (int k = 10; k < 18; ++k)
       if (nt[k] >= ((int64_t)1 << 31)) return bad(BLDFM_ELIMIT, "too many four-step transforms in one instance");
     for (int k = 0; k < kKinds; ++k) tiles[k][i + 1] = tiles[k][i] + nt[k];
+  }
+  // The march in pairs of modes (k_shoot_pair) does 155 operations a step for
+  // two modes instead of 2 x 84 but has half the waves: it is taken where the
+  // plan's waves fill the 1024 SIMDs often enough.  A lone 512^2 footprint (2057
+  // waves, 3 rounds of 84, or 1040 pair waves, 2 rounds of 155) keeps one mode a
+  // lane; a batch of 128 of them takes pairs.
+  auto pairs = [](const InstDesc& D) { return D.exact && (D.variant == 0 || D.variant == 2); };
+  int64_t waves[2] = {0, 0};
+  for (const InstDesc& D : P->desc) {
+    waves[0] += (D.lanes + 63) / 64;
+    waves[1] += ((pairs(D) ? D.plane : D.lanes) + 63) / 64;
+  }
+  const bool by_pair = (waves[1] + 1023) / 1024 * 155 < (waves[0] + 1023) / 1024 * 84;
+  int pair_used[4] = {0, 0, 0, 0};
+  for (int i = 0; i < ninst; ++i) {
+    InstDesc& D = P->desc[i];
+    D.pair = by_pair && pairs(D);
+    (D.pair ? pair_used[D.variant] : variant_used[D.variant][D.exact]) = 1;
+    tiles[3][i + 1] = tiles[3][i] + ((D.pair ? D.plane : D.lanes) + shoot_block - 1) / shoot_block;
   }
   if (lv - levels > (int64_t)1 << 31) return bad(BLDFM_EINVAL, "level table too large");
   P->setups = met;
@@ -847,6 +866,7 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
   V.any_dispersion = any_disp;
   for (int k = 0; k < 4; ++k)
     for (int e = 0; e < 2; ++e) V.variant_used[k][e] = variant_used[k][e];
+  for (int k = 0; k < 4; ++k) V.pair_used[k] = pair_used[k];
   V.fft_small = fft_small;
   V.fft_threads = fft_threads;
   V.fft_lds_bytes = fft_lds_bytes(max_n);  // non-decreasing in n

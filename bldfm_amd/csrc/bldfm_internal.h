@@ -29,6 +29,7 @@ struct PlanDev {
   int32_t ninst;
   int32_t any_dispersion;
   int32_t variant_used[4][2]; // shooting kernels this plan launches [variant][exact]
+  int32_t pair_used[4];       // k_shoot_pair by variant
   int32_t fft_small;       // all transforms <= BLDFM_FFT_SMALL_N: 256-thread kernels
   int32_t fft_threads;     // threads per FFT workgroup
   int32_t fft_lds_bytes;   // dynamic LDS per FFT workgroup

@@ -26,7 +26,7 @@
 //           them: sa = 0.5*kappa, h2 = h*h, b0 = (-kappa)*h,
 //           sb = (1/6)*(kappa*kappa), h3 = h*(h*h), h, sc = (1/6)*kappa,
 //           W = 0.5/Kz_i + 0.5/Kz_{i+1}  (trapezoid weight of the (0,0) mode)
-//   [12..14] fused-path coefficients A = sa*h2, B1 = sb*h3, C = sc*h3
+//   [12..14] fused-path coefficients A = sa*h2, B1 = sb*h3, C = sc*h3; [15] 2 sc
 // so that T = -(Kx lx^2 + Ky ly^2) - i(u lx + v ly), a = d = 1 - sa T h2,
 // b = b0 - sb T h3, c = T h - sc T^2 h3.
 // Entry nz-1 (top, src/bldfm/solver.py:164-174):
@@ -59,7 +59,7 @@ __device__ __forceinline__ void fill_level_row(const double* cur, const double* 
     T[12] = sa * h2;
     T[13] = sb * h3;
     T[14] = sc * h3;
-    T[15] = 0.0;
+    T[15] = sc + sc;
   } else {
     T[0] = cur[3] * kinv;
     T[1] = cur[4] * kinv;
@@ -156,11 +156,11 @@ __device__ void origin_numeric(const cdesc_t& D, const double* __restrict__ tab,
 // march from the bottom after the shooting coefficient is known
 // (RECOMP == true) for many output levels.  Both give the same values.
 template <int MAXS, bool RECOMP, bool EXACT, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_shoot(PlanDev P, ExecBufs B, int variant) {
+__global__ __launch_bounds__(BLOCK, MAXS == 1 ? 5 : 3) void k_shoot(PlanDev P, ExecBufs B, int variant) {
   for (int64_t t = blockIdx.x; t < P.tot_shoot; t += gridDim.x) {
     const TileRec tr = tile_rec(P.t_shoot, t);
     const cdesc_t& D = *(const cdesc_t*)(P.desc + tr.inst);
-    if (D.variant != variant || D.exact != (int)EXACT) continue;
+    if (D.variant != variant || D.exact != (int)EXACT || D.pair) continue;
     if (B.mode && B.mode[tr.inst] == 0) continue;  // accepted surrogate instance
     Lane L;
     const int lane = tr.local * BLOCK + (int)threadIdx.x;
@@ -227,6 +227,110 @@ __global__ __launch_bounds__(BLOCK) void k_shoot(PlanDev P, ExecBufs B, int vari
       }
     }
     for (int s = D.nfilled; s < D.nslot; ++s) emit_mode(D, L, B.ws, s, cmk(0.0, 0.0), cmk(0.0, 0.0), sh);
+  }
+}
+
+// The numerical branch with a mode and its mirror in x per lane (exact
+// rounding; one register snapshot, or the second march).  The march is bound
+// by FP64 issue (95% of the slots) and by the clock the card holds under it,
+// so the operations that a pair shares are its gain: 128 footprints of 512^2 x
+// 64 take 1.44e9 vector instructions instead of 1.57e9 and 10% fewer cycles, of
+// which the lower clock (1.83 against 1.99 GHz) takes half: 2.74 -> 2.64 ms.
+template <bool RECOMP, int BLOCK>
+__global__ __launch_bounds__(BLOCK, 4) void k_shoot_pair(PlanDev P, ExecBufs B, int variant) {
+  for (int64_t t = blockIdx.x; t < P.tot_shoot; t += gridDim.x) {
+    const TileRec tr = tile_rec(P.t_shoot, t);
+    const cdesc_t& D = *(const cdesc_t*)(P.desc + tr.inst);
+    if (D.variant != variant || !D.pair) continue;
+    if (B.mode && B.mode[tr.inst] == 0) continue;  // accepted surrogate instance
+    const int lane = tr.local * BLOCK + (int)threadIdx.x;
+    const double* __restrict__ tab = B.tab + D.off_tab;
+    const int wave0 = __builtin_amdgcn_readfirstlane(lane);
+    const int o = pair_origin_lane(D.nlx, D.nly) - wave0;
+    if (o >= 0 && o < 64) origin_numeric(D, tab, P.ints + D.off_slot, B.ws);
+    if (lane >= D.plane) continue;
+    Lane L;
+    L.fx = L.fy = 0;
+    int two, nidx2;
+    L.kind = decode_pair(lane, D.nlx, D.nly, &L.fx, &L.fy, &L.nidx, &two, &nidx2);
+    if (L.kind == LANE_IDLE || L.kind == LANE_ORIGIN) continue;
+    L.lx = xmul(D.sx, xmul((double)L.fx, D.vx));
+    L.ly = xmul(D.sy, xmul((double)L.fy, D.vy));
+    Lane L2 = L;
+    if (two) {
+      L2.fx = -L.fx;
+      L2.lx = -L.lx;
+      L2.nidx = nidx2;
+    }
+    ctab_t* __restrict__ ctab = (ctab_t*)tab;
+    cint_t* __restrict__ slot = (cint_t*)(P.ints + D.off_slot);
+    const int nz = D.nz;
+    const double lx = L.lx, ly = L.ly, lx2 = xmul(lx, lx), ly2 = xmul(ly, ly);
+    const double2 one = cmk(1.0, 0.0), zero = cmk(0.0, 0.0);
+    double2 p1[2] = {one, one}, q1[2] = {zero, zero}, p2[2] = {zero, zero};
+    double2 q2[2] = {ivp2_init(D, L, B.ws), ivp2_init(D, L2, B.ws)};
+    double2 sp1[2], sq1[2], sp2[2], sq2[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) sp1[m] = sq1[m] = sp2[m] = sq2[m] = zero;
+    const int snap = D.snap_level[0];
+    Row nxt = load_row(ctab);
+#pragma unroll 2
+    for (int i = 0; i < nz - 1; ++i) {
+      if (!RECOMP && i == snap) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m) { sp1[m] = p1[m]; sq1[m] = q1[m]; sp2[m] = p2[m]; sq2[m] = q2[m]; }
+      }
+      const Row cur = nxt;
+      if (i + 1 < nz - 1) nxt = load_row(ctab + (int64_t)(i + 1) * BLDFM_LEVEL_STRIDE);
+      march_pair(cur, lx, ly, lx2, ly2, p1, q1, p2, q2);
+    }
+    if (!RECOMP && nz - 1 == snap) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) { sp1[m] = p1[m]; sq1[m] = q1[m]; sp2[m] = p2[m]; sq2[m] = q2[m]; }
+    }
+    const double* tt = tab + (int64_t)(nz - 1) * BLDFM_LEVEL_STRIDE;
+    double2 alpha[2], sh[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const Lane& M = m ? L2 : L;
+      alpha[m] = shoot_alpha(tt, top_lambda(tt, M.lx, M.ly, lx2, ly2), p1[m], q1[m], p2[m], q2[m]);
+      sh[m] = phase_shift(D, M);
+    }
+    if (!RECOMP) {
+      if (D.nfilled > 0) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          if (m == 0 || two)
+            emit_mode(D, m ? L2 : L, B.ws, 0, xcadd(ncmul(alpha[m], sp1[m]), sp2[m]),
+                      xcadd(ncmul(alpha[m], sq1[m]), sq2[m]), sh[m]);
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        p1[m] = one; q1[m] = zero; p2[m] = zero;
+        q2[m] = ivp2_init(D, m ? L2 : L, B.ws);
+      }
+      Row nxt2 = load_row(ctab);
+      for (int i = 0; i <= D.max_level; ++i) {
+        const int sl = slot[i];
+        if (sl >= 0) {
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+            if (m == 0 || two)
+              emit_mode(D, m ? L2 : L, B.ws, sl, xcadd(ncmul(alpha[m], p1[m]), p2[m]),
+                        xcadd(ncmul(alpha[m], q1[m]), q2[m]), sh[m]);
+        }
+        if (i < D.max_level) {
+          const Row cur = nxt2;
+          if (i + 1 < D.max_level) nxt2 = load_row(ctab + (int64_t)(i + 1) * BLDFM_LEVEL_STRIDE);
+          march_pair(cur, lx, ly, lx2, ly2, p1, q1, p2, q2);
+        }
+      }
+    }
+    for (int s = D.nfilled; s < D.nslot; ++s)
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        if (m == 0 || two) emit_mode(D, m ? L2 : L, B.ws, s, zero, zero, sh[m]);
   }
 }
 
@@ -550,6 +654,16 @@ int bldfm_launch_all(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int
   SHOOT(1, 4, false, false)
   SHOOT(2, 1, true, false)
 #undef SHOOT
+#define SHOOT_PAIR(V, RECOMP)                                                             \
+  if (P.pair_used[V]) {                                                                   \
+    if (P.shoot_block == 64) k_shoot_pair<RECOMP, 64><<<gs, 64, 0, stream>>>(P, B, V);    \
+    else if (P.shoot_block == 128) k_shoot_pair<RECOMP, 128><<<gs, 128, 0, stream>>>(P, B, V); \
+    else k_shoot_pair<RECOMP, 256><<<gs, 256, 0, stream>>>(P, B, V);                      \
+    LAUNCH_CHECK();                                                                       \
+  }
+  SHOOT_PAIR(0, false)
+  SHOOT_PAIR(2, true)
+#undef SHOOT_PAIR
   if (P.variant_used[3][0] || P.variant_used[3][1]) {
     if (P.shoot_block == 64) k_shoot_analytic<64><<<gs, 64, 0, stream>>>(P, B, 3);
     else if (P.shoot_block == 128) k_shoot_analytic<128><<<gs, 128, 0, stream>>>(P, B, 3);

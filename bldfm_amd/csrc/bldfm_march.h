@@ -111,14 +111,14 @@ typedef const __attribute__((address_space(4))) int32_t cint_t;
 
 // One level-table row in registers (SGPRs: the row is uniform).
 struct Row {
-  double kx, ky, u, v, sa, h2, b0, sb, h3, h, sc, A, B1, C;
+  double kx, ky, u, v, sa, h2, b0, sb, h3, h, sc, A, B1, C, sc2;
 };
 
 __device__ __forceinline__ Row load_row(ctab_t* __restrict__ T) {
   Row r;
   r.kx = T[0]; r.ky = T[1]; r.u = T[2]; r.v = T[3];
   r.sa = T[4]; r.h2 = T[5]; r.b0 = T[6]; r.sb = T[7]; r.h3 = T[8]; r.h = T[9]; r.sc = T[10];
-  r.A = T[12]; r.B1 = T[13]; r.C = T[14];
+  r.A = T[12]; r.B1 = T[13]; r.C = T[14]; r.sc2 = T[15];
   return r;
 }
 
@@ -136,15 +136,42 @@ __device__ __forceinline__ void march_step<true>(const Row& R, double lx, double
   const double ar = 1.0 - (R.sa * tr) * R.h2, ai = -((R.sa * ti) * R.h2);
   const double br = R.b0 - (R.sb * tr) * R.h3, bi = -((R.sb * ti) * R.h3);
   const double t2r = tr * tr - ti * ti;
-  const double tri = tr * ti;
-  const double t2i = tri + tri;
-  const double cr = tr * R.h - (R.sc * t2r) * R.h3, ci = ti * R.h - (R.sc * t2i) * R.h3;
+  // sc * (tri + tri) = (2 sc) * tri: doubling commutes with the rounding
+  const double cr = tr * R.h - (R.sc * t2r) * R.h3, ci = ti * R.h - (R.sc2 * (tr * ti)) * R.h3;
   const double2 a = cmk(ar, ai), b = cmk(br, bi), c = cmk(cr, ci);
   const double2 np1 = xcmuladd(a, p1, b, q1);
   const double2 nq1 = xcmuladd(c, p1, a, q1);
   const double2 np2 = xcmuladd(a, p2, b, q2);
   const double2 nq2 = xcmuladd(c, p2, a, q2);
   p1 = np1; q1 = nq1; p2 = np2; q2 = nq2;
+}
+
+// One exact step of the modes (lx, ly) and (-lx, ly): the same roundings as
+// two march_step<true>, with what does not depend on the sign of lx -- the
+// real part of T and all it enters, and the products u lx, v ly -- formed
+// once: 155 operations instead of 168.
+__device__ __forceinline__ void march_pair(const Row& R, double lx, double ly, double lx2, double ly2, double2 (&p1)[2],
+                                           double2 (&q1)[2], double2 (&p2)[2], double2 (&q2)[2]) {
+#pragma clang fp contract(off)
+  const double tr = -(R.kx * lx2 + R.ky * ly2);
+  const double ul = R.u * lx, vl = R.v * ly;
+  const double ti[2] = {-(ul + vl), -(vl - ul)};
+  const double ar = 1.0 - (R.sa * tr) * R.h2;
+  const double br = R.b0 - (R.sb * tr) * R.h3;
+  const double trh = tr * R.h, tr2 = tr * tr;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const double ai = -((R.sa * ti[m]) * R.h2);
+    const double bi = -((R.sb * ti[m]) * R.h3);
+    const double t2r = tr2 - ti[m] * ti[m];
+    const double cr = trh - (R.sc * t2r) * R.h3, ci = ti[m] * R.h - (R.sc2 * (tr * ti[m])) * R.h3;
+    const double2 a = cmk(ar, ai), b = cmk(br, bi), c = cmk(cr, ci);
+    const double2 np1 = xcmuladd(a, p1[m], b, q1[m]);
+    const double2 nq1 = xcmuladd(c, p1[m], a, q1[m]);
+    const double2 np2 = xcmuladd(a, p2[m], b, q2[m]);
+    const double2 nq2 = xcmuladd(c, p2[m], a, q2[m]);
+    p1[m] = np1; q1[m] = nq1; p2[m] = np2; q2[m] = nq2;
+  }
 }
 
 template <>

@@ -164,6 +164,7 @@ struct InstDesc {
   int64_t off_long;     // workspace double2: four-step scratch (lines x n of the longest split pass)
   int32_t long_x, long_y;  // 1: the padded x / y length is split (four-step passes)
   LineAlg line[4];         // forward rows, forward columns, inverse y-pass, inverse x-pass
+  int32_t pair, plane;     // 1: marched by k_shoot_pair; its lanes
   int32_t nyq_direct;      // 1: every Nyquist mode's mirror is outside the retained modes
 };
 
@@ -261,6 +262,78 @@ BLDFM_HD int decode_lane(int lane, int nlx, int nly, int* fx, int* fy, int* nidx
       *nidx = (nly % 2 == 0 ? nlx : 0) + lane;
       return LANE_NYQ;
     }
+  }
+  return LANE_IDLE;
+}
+
+// Shooting lanes that march a mode and its mirror in x together, (fx, fy) and
+// (-fx, fy) with fx > 0: the upper half plane, then the Nyquist row; then the
+// modes without such a partner (fx = 0, fy = 0, the origin, the rest of the
+// Nyquist modes), one per lane.
+BLDFM_HD int pair_lanes(int nlx, int nly) {
+  const int Px = paired_max(nlx), Py = paired_max(nly);
+  return Px * Py + (nly % 2 ? 0 : Px) + Py + Px + 1 + (nly % 2 ? 0 : 2 - nlx % 2) + (nlx % 2 ? 0 : 2 * Py + 1);
+}
+BLDFM_HD int pair_origin_lane(int nlx, int nly) {
+  const int Px = paired_max(nlx), Py = paired_max(nly);
+  return Px * Py + (nly % 2 ? 0 : Px) + Py + Px;
+}
+// As decode_lane; *two: the lane also holds (-fx, fy), with Nyquist index *nidx2.
+BLDFM_HD int decode_pair(int lane, int nlx, int nly, int* fx, int* fy, int* nidx, int* two, int* nidx2) {
+  const int Px = paired_max(nlx), Py = paired_max(nly);
+  *nidx = *nidx2 = -1;
+  *two = 1;
+  if (lane < 0) return LANE_IDLE;
+  if (lane < Px * Py) {
+    *fx = lane / Py + 1;
+    *fy = lane % Py + 1;
+    return LANE_HALF;
+  }
+  lane -= Px * Py;
+  if (nly % 2 == 0) {
+    if (lane < Px) {
+      *fx = lane + 1;
+      *fy = -nly / 2;
+      *nidx = trunc_of_freq(lane + 1, nlx);
+      *nidx2 = trunc_of_freq(-(lane + 1), nlx);
+      return LANE_NYQ;
+    }
+    lane -= Px;
+  }
+  *two = 0;
+  if (lane < Py) {
+    *fx = 0;
+    *fy = lane + 1;
+    return LANE_HALF;
+  }
+  lane -= Py;
+  if (lane < Px) {
+    *fx = lane + 1;
+    *fy = 0;
+    return LANE_HALF;
+  }
+  lane -= Px;
+  if (lane == 0) {
+    *fx = 0;
+    *fy = 0;
+    return LANE_ORIGIN;
+  }
+  lane -= 1;
+  if (nly % 2 == 0) {
+    const int n = 2 - nlx % 2;
+    if (lane < n) {
+      *fx = lane == 0 ? 0 : -nlx / 2;
+      *fy = -nly / 2;
+      *nidx = trunc_of_freq(*fx, nlx);
+      return LANE_NYQ;
+    }
+    lane -= n;
+  }
+  if (nlx % 2 == 0 && lane < 2 * Py + 1) {
+    *fx = -nlx / 2;
+    *fy = lane - Py;
+    *nidx = (nly % 2 == 0 ? nlx : 0) + lane;
+    return LANE_NYQ;
   }
   return LANE_IDLE;
 }

@@ -181,3 +181,13 @@ def test_nyquist_direct_emission(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout
     assert int(out.stdout.split()[2]) > 100, out.stdout
+
+
+def test_pair_lanes(tmp_path):
+    """Compile tests/native/pair_lanes_check.cpp: the lanes that march two
+    modes cover the modes of the one-mode lanes exactly once."""
+    exe = tmp_path / "pair_lanes_check"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-o", str(exe),
+                    str(ROOT / "tests" / "native" / "pair_lanes_check.cpp")], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
