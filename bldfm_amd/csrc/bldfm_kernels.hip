@@ -71,34 +71,76 @@ __device__ __forceinline__ void fill_level_row(const double* cur, const double* 
   }
 }
 
-__global__ __launch_bounds__(256) void k_level_table(PlanDev P, ExecBufs B) {
+// Profiles of up to 256 levels i0 + tid by a workgroup of 4 x 256 threads,
+// same values as prof_point.  A level's correctly rounded functions are one
+// long serial chain (about nine logarithms), and a plan has few levels, so the
+// four groups evaluate what does not depend on each other: z, then log(z/z0),
+// xi and phi, then psi's two logarithms and its arctangent; the chain is about
+// half as long.  A wave issues one of its dependent FP64 operations every eight
+// cycles, so the groups' waves of the same levels go to different SIMDs
+// (on one SIMD they took as long as one wave): the unstable profiles of 26
+// levels take 12.5 us instead of 27, k_level_table of 96 footprints 16.4 instead
+// of 32.7.
+// Leaves out = {z, u, v, Kx, Ky, Kz} in the registers of group 0.
+struct GroupSlot {
+  int grp, tid;
+};
+__device__ __forceinline__ GroupSlot group_slot() {
+  const int wave = (int)threadIdx.x >> 6, grp = wave >> 2;  // wave w runs on SIMD w mod 4
+  return GroupSlot{grp, ((wave + grp) & 3) * 64 + (int)(threadIdx.x & 63)};
+}
+__device__ __forceinline__ void prof_group(const ProfSetup& S, int i, bool live, double (*sh)[256], double out[6]) {
+#pragma clang fp contract(off)
+  const int tid = group_slot().tid, grp = group_slot().grp;
+  const bool most = S.closure == CL_MOST || S.closure == CL_MOSTM;
+  __syncthreads();  // the last call's values are read
+  if (grp == 0 && live) sh[0][tid] = prof_z(S, i);
+  __syncthreads();
+  const double z = sh[0][tid], x = z / S.mol;
+  if (live && S.closure != CL_CONSTANT) {
+    if (grp == 0) sh[1][tid] = cr_log(z / S.z0);
+    if (most && grp == 1 && !(x > 0.0)) sh[2][tid] = gl_cpow_real(1.0 - 16.0 * x, 0.25);
+    if (most && grp == 2) sh[3][tid] = most_phi(x);
+  }
+  __syncthreads();
+  if (live && most && !(x > 0.0)) {
+    const double xi = sh[2][tid];
+    if (grp == 1) sh[4][tid] = cr_log(0.5 * (1.0 + xi));
+    if (grp == 2) sh[5][tid] = cr_log(0.5 * (1.0 + xi * xi));
+    if (grp == 3) sh[6][tid] = cr_atan(xi);
+  }
+  __syncthreads();
+  if (grp == 0 && live)
+    prof_combine(S, z, sh[1][tid], x > 0.0 ? 5.0 * x : psi_of(sh[4][tid], sh[5][tid], sh[6][tid]), sh[3][tid], out);
+}
+
+__global__ __launch_bounds__(1024) void k_level_table(PlanDev P, ExecBufs B) {
 #pragma clang fp contract(off)
   // levels evaluated from met in this tile: 256 of them and the one above
   __shared__ double lev[6][257];
+  __shared__ double sh[7][256];
   for (int64_t t = blockIdx.x; t < P.tot_tab; t += gridDim.x) {
     const TileRec tr = tile_rec(P.t_tab, t);
     const int inst = tr.inst;
     const cdesc_t& D = *(const cdesc_t*)(P.desc + inst);
     const int nz = D.nz;
-    const int tid = (int)threadIdx.x, T = (int)blockDim.x;
-    const int i = tr.local * T + tid;
+    const int tid = group_slot().tid, grp = group_slot().grp;
+    const int i = tr.local * 256 + tid;
     double* prof = B.prof + D.off_prof;
     double cur[6], nxt[6];
     if (P.met_flag[inst]) {  // uniform over the workgroup (one instance per tile)
-      // every level once (the correctly rounded profile functions are the
-      // costly part): each thread its level, the last thread also the next
+      // every level once: group 0 its level, and where the tile ends inside the
+      // grid one thread of group 3 the next tile's first
       const ProfSetup& S = P.met[inst];
-      if (t != blockIdx.x) __syncthreads();  // the previous tile's reads of lev are done
-      if (i < nz) {
-        prof_point(S, i, cur);
+      prof_group(S, i, i < nz, sh, cur);
+      if (grp == 0 && i < nz)
         for (int c = 0; c < 6; ++c) {
           prof[(int64_t)c * nz + i] = cur[c];
           lev[c][tid] = cur[c];
         }
-      }
-      if (tid == T - 1 && i + 1 < nz) {
+      if (grp == 3 && tid == 255 && i + 1 < nz) {
         prof_point(S, i + 1, nxt);
-        for (int c = 0; c < 6; ++c) lev[c][T] = nxt[c];
+        for (int c = 0; c < 6; ++c) lev[c][256] = nxt[c];
       }
       __syncthreads();
       if (i + 1 < nz)
@@ -109,7 +151,8 @@ __global__ __launch_bounds__(256) void k_level_table(PlanDev P, ExecBufs B) {
       if (i + 1 < nz)
         for (int c = 0; c < 6; ++c) nxt[c] = prof[(int64_t)c * nz + i + 1];
     }
-    if (i < nz) fill_level_row(cur, nxt, i == nz - 1, B.tab + D.off_tab + (int64_t)i * BLDFM_LEVEL_STRIDE);
+    if (grp == 0 && i < nz)
+      fill_level_row(cur, nxt, i == nz - 1, B.tab + D.off_tab + (int64_t)i * BLDFM_LEVEL_STRIDE);
   }
 }
 
@@ -605,7 +648,7 @@ int bldfm_launch_all(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int
   }
   MARK(0)
   if (P.tot_tab > 0) {
-    k_level_table<<<grid_for(P.tot_tab, grid_cap), 256, 0, stream>>>(P, B);
+    k_level_table<<<grid_for(P.tot_tab, grid_cap), 1024, 0, stream>>>(P, B);
     LAUNCH_CHECK();
   }
   MARK(1)
@@ -692,16 +735,17 @@ int bldfm_launch_all(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int
 // ---------------------------------------------------------------- profiles
 // Array part of vertical_profiles (src/bldfm/pbl_model.py:127-182):
 // out = [z | u | v | Kx | Ky | Kz], nlev each.
-__global__ __launch_bounds__(256) void k_profiles(ProfSetup S, double* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= S.nlev) return;
+__global__ __launch_bounds__(1024) void k_profiles(ProfSetup S, double* __restrict__ out) {
+  __shared__ double sh[7][256];
+  const int i = blockIdx.x * 256 + group_slot().tid;
   double o[6];
-  prof_point(S, i, o);
-  for (int c = 0; c < 6; ++c) out[(int64_t)c * S.nlev + i] = o[c];
+  prof_group(S, i, i < S.nlev, sh, o);
+  if (group_slot().grp == 0 && i < S.nlev)
+    for (int c = 0; c < 6; ++c) out[(int64_t)c * S.nlev + i] = o[c];
 }
 
 int bldfm_launch_profiles(const ProfSetup& S, double* out, hipStream_t stream) {
-  k_profiles<<<(S.nlev + 255) / 256, 256, 0, stream>>>(S, out);
+  k_profiles<<<(S.nlev + 255) / 256, 1024, 0, stream>>>(S, out);
   LAUNCH_CHECK();
   return 0;
 }

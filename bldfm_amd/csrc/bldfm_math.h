@@ -169,6 +169,12 @@ template <bool EXACT> BLDFM_HD double pf_cpow(double v, double p) {
   return EXACT ? gl_cpow_real(v, p) : exp(p * log(v));
 }
 
+// psi for x <= 0 from its three function values.
+BLDFM_HD double psi_of(double log1, double log2, double at) {
+  CR_EXACT
+  return -2.0 * log1 - log2 + 2.0 * at - 0.5 * BLDFM_PI;
+}
+
 // MOST momentum stability correction psi(z/L) (src/bldfm/pbl_model.py:207-230):
 // 5x for x > 0, else with xi = Re((1 - 16x)^(1/4)) (complex power)
 // -2 ln((1 + xi)/2) - ln((1 + xi^2)/2) + 2 atan(xi) - pi/2.
@@ -177,8 +183,7 @@ BLDFM_HD double most_psi(double x) {
   CR_EXACT
   if (x > 0.0) return 5.0 * x;
   const double xi = pf_cpow<EXACT>(1.0 - 16.0 * x, 0.25);
-  return -2.0 * pf_log<EXACT>(0.5 * (1.0 + xi)) - pf_log<EXACT>(0.5 * (1.0 + xi * xi)) + 2.0 * pf_atan<EXACT>(xi) -
-         0.5 * BLDFM_PI;
+  return psi_of(pf_log<EXACT>(0.5 * (1.0 + xi)), pf_log<EXACT>(0.5 * (1.0 + xi * xi)), pf_atan<EXACT>(xi));
 }
 
 // MOST diffusivity stability function phi(z/L) (src/bldfm/pbl_model.py:233-250).
@@ -275,23 +280,28 @@ BLDFM_HD int prof_setup_given(int n, double zm, double um, double vm, double ust
   return 0;
 }
 
-// Height and profile values at grid point i (src/bldfm/pbl_model.py:127-182).
-// out = {z, u, v, Kx, Ky, Kz}
+// Height of grid point i (src/bldfm/pbl_model.py:127-129).
 template <bool EXACT = true>
-BLDFM_HD void prof_point(const ProfSetup& s, int i, double out[6]) {
+BLDFM_HD double prof_z(const ProfSetup& s, int i) {
+  CR_EXACT
+  const double zeta = 0.0 + i * s.dzeta;
+  return -s.h * pf_log<EXACT>(-(zeta - s.aa) / s.bb);
+}
+
+// Profile values at height z from log(z/z0), psi(z/L) and phi(z/L) (each read
+// only by the closures that use it).  out = {z, u, v, Kx, Ky, Kz}
+BLDFM_HD void prof_combine(const ProfSetup& s, double z, double logz, double psi, double phi, double out[6]) {
   CR_EXACT
   const double kap = BLDFM_KARMAN;
-  const double zeta = 0.0 + i * s.dzeta;
-  const double z = -s.h * pf_log<EXACT>(-(zeta - s.aa) / s.bb);
   double u, v, kx, ky, kz;
   if (s.closure == CL_CONSTANT) {
     const double km = kap * s.ustar * s.zm / s.prsc;
     u = s.um; v = s.vm; kx = ky = kz = km;
   } else if (s.closure == CL_MOST || s.closure == CL_MOSTM) {
-    const double absu = s.ustar / kap * (pf_log<EXACT>(z / s.z0) + most_psi<EXACT>(z / s.mol));
+    const double absu = s.ustar / kap * (logz + psi);
     u = s.um / s.absum * absu;
     v = s.vm / s.absum * absu;
-    const double K = kap * s.ustar * z / most_phi<EXACT>(z / s.mol) / s.prsc;
+    const double K = kap * s.ustar * z / phi / s.prsc;
     if (s.closure == CL_MOST) {
       kx = ky = kz = K;
     } else {
@@ -301,10 +311,19 @@ BLDFM_HD void prof_point(const ProfSetup& s, int i, double out[6]) {
     }
   } else {  // OAAHOC
     const double cl = 0.845, cm = 0.0856, ch = 0.204;
-    const double absu = s.ustar * s.ustar / cm / cl / sqrt(s.tke) * pf_log<EXACT>(z / s.z0);
+    const double absu = s.ustar * s.ustar / cm / cl / sqrt(s.tke) * logz;
     u = s.um / s.absum * absu;
     v = s.vm / s.absum * absu;
     kx = ky = kz = ch * cl * z * sqrt(s.tke);
   }
   out[0] = z; out[1] = u; out[2] = v; out[3] = kx; out[4] = ky; out[5] = kz;
+}
+
+// Height and profile values at grid point i (src/bldfm/pbl_model.py:127-182).
+template <bool EXACT = true>
+BLDFM_HD void prof_point(const ProfSetup& s, int i, double out[6]) {
+  const double z = prof_z<EXACT>(s, i);
+  const bool most = s.closure == CL_MOST || s.closure == CL_MOSTM;
+  prof_combine(s, z, s.closure == CL_CONSTANT ? 0.0 : pf_log<EXACT>(z / s.z0), most ? most_psi<EXACT>(z / s.mol) : 0.0,
+               most ? most_phi<EXACT>(z / s.mol) : 1.0, out);
 }
