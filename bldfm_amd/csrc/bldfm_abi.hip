@@ -1219,7 +1219,11 @@ int bldfm_sur_train_grad(const void* net, const float* surmet, int32_t nmet, con
   rc = bldfm_launch_sur_forward((const uint8_t*)net, (const SurMet*)surmet, nmet, blk_met, (const double2*)kxy,
                                 (const double2*)g, npts, xs, zs, dphi, (float2*)phi, loss, 1, stream);
   if (rc) return launch_fail(rc, "surrogate forward");
-  const int chunk = npts % 2048 == 0 ? 2048 : SUR_PTS;
+  // points per workgroup of the weight gradients: 18 workgroups a chunk, so 64
+  // chunks give each CU four or five (65,536 points: 4096, 2048, 1024 and 512 a
+  // chunk take 191, 141, 111 and 149 us), each with 16384 atomic additions at its end
+  int chunk = 2048;
+  while (chunk > SUR_PTS && (npts % chunk || npts / chunk < 64)) chunk /= 2;
   rc = bldfm_launch_sur_backward((const uint8_t*)net, npts, xs, zs, dphi, dzs, grad, chunk, stream);
   return rc ? launch_fail(rc, "surrogate backward") : 0;
 }

@@ -57,7 +57,10 @@ __device__ __forceinline__ int64_t xs_off(int l, int64_t N) {
 // weight gradient sums over points, in any order; the inputs x_0 keep the
 // points' order and are brought to the others' as they are staged.)  z_l is read back by the same
 // lanes only and is kept in accumulator order (zs_off), 512 bytes a store.
-// Forward 158 -> 148 us, backward 304 -> 179 us at 65,536 points.
+// These layouts took the forward from 158 to 148 us and the backward from 304 to
+// 179 at 65,536 points, and loads ahead of their use (sur_hidden's U, fetch_z,
+// k_sur_wgrad's fetch) to 113 and 127, the weight gradients from 189 to 110; the
+// floor is their 350 MB each, 66 us at the rate of a large copy.
 __device__ __forceinline__ int sur_pt_at(int pos) { return ((pos & 3) << 5) | (pos >> 2); }
 __device__ __forceinline__ int64_t zs_off(int l, int64_t N, int64_t p0, int wave, int a, int jq, int pb, int lane) {
   return ((((((int64_t)l * (N / SUR_PTS) + p0 / SUR_PTS) * 4 + wave) * 2 + a) * 4 + jq) * 4 + pb) * 256 + lane * 4;
@@ -288,7 +291,9 @@ __device__ __forceinline__ void sur_hidden(const uint8_t* __restrict__ net, cons
                                            __bf16* __restrict__ xs, __bf16* __restrict__ zs, int64_t N,
                                            int64_t p0) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  constexpr int U = TRAIN ? 1 : SUR_W / 32;  // the training kernel has no registers to spare
+  // the training kernel is fastest with the next step's weights under this step's
+  // products (113 us at 65,536 points; 148 without, 119 with four or eight steps)
+  constexpr int U = TRAIN ? 2 : SUR_W / 32;
   f32x16 acc[2][4];
   // layer 0, the middle layers and the last layer as straight-line code: with
   // the epilogue kinds in branches of one loop body the compiler hoists their
@@ -510,7 +515,17 @@ __global__ __launch_bounds__(SUR_THREADS, 2) void k_sur_bwd(const uint8_t* __res
   bias_grad(act, part, grad + SUR_P_B(SUR_NL - 1));
   f32x16 acc[2][4];
   for (int l = SUR_NL - 1; l >= 1; --l) {
-    mfma_tile<SUR_W / 16, SUR_W / 16>((const bf16x8*)(net + SUR_OFF_WT(l)), act, wave, lane, acc);
+    // z of the lower half of this wave's features is fetched under the products,
+    // that of the upper half under the lower half's epilogue
+    bf16x4 zf[2][16];
+    auto fetch_z = [&](int a) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q)
+        zf[a][q] = *(const bf16x4*)(zs + zs_off(l - 1, N, p0, wave, a, q >> 2, q & 3, lane));
+    };
+    fetch_z(0);
+    mfma_tile<SUR_W / 16, 2>((const bf16x8*)(net + SUR_OFF_WT(l)), act, wave, lane, acc);
+    fetch_z(1);
     __syncthreads();
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
@@ -521,7 +536,7 @@ __global__ __launch_bounds__(SUR_THREADS, 2) void k_sur_bwd(const uint8_t* __res
 #pragma unroll
         for (int pb = 0; pb < 4; ++pb) {
           const int pt = 32 * pb + r;
-          const bf16x4 z = *(const bf16x4*)(zs + zs_off(l - 1, N, p0, wave, a, jq, pb, lane));
+          const bf16x4 z = zf[a][jq * 4 + pb];
           float v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -583,28 +598,41 @@ __global__ __launch_bounds__(SUR_THREADS, 2) void k_sur_wgrad(int64_t N, int chu
 #pragma unroll
   for (int i = 0; i < 8; ++i) zero[i] = (__bf16)0.0f;
   const int64_t pbeg = (int64_t)c * chunk, pend = pbeg + chunk;
-  for (int64_t p = pbeg; p < pend; p += WG_PSTEP) {
-    for (int q = tid; q < 128 * (WG_PSTEP / 8); q += SUR_THREADS) {
-      const int row = q / (WG_PSTEP / 8), ch = q % (WG_PSTEP / 8);
-      const int so = row * WG_PSTEP + ((ch ^ (row & 7)) << 3);
-      *(bf16x8*)(sa + so) = *(const bf16x8*)(dZ + (int64_t)(ot * 128 + row) * N + p + ch * 8);
+  // the next step's operands are on their way to registers while this step's
+  // products run (189 -> 141 us at 65,536 points in chunks of 2048)
+  bf16x8 ra[4], rb[4];
+  auto fetch = [&](int64_t p) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int q = tid + k * SUR_THREADS, row = q / (WG_PSTEP / 8), ch = q % (WG_PSTEP / 8);
+      ra[k] = *(const bf16x8*)(dZ + (int64_t)(ot * 128 + row) * N + p + ch * 8);
       const int krow = kt * 128 + row;
-      bf16x8 xv = zero;
+      rb[k] = zero;
       if (krow < kin && l > 0) {
-        xv = *(const bf16x8*)(X + (int64_t)krow * N + p + ch * 8);
-      } else if (krow < kin) {  // positions q .. q + 7: points q/4 and q/4 + 1 of each quarter of the block
-        const int q = (int)(p % SUR_PTS) + ch * 8;
-        const __bf16* xr = X + (int64_t)krow * N + p / SUR_PTS * SUR_PTS + (q >> 2);
+        rb[k] = *(const bf16x8*)(X + (int64_t)krow * N + p + ch * 8);
+      } else if (krow < kin) {  // positions s .. s + 7: points s/4 and s/4 + 1 of each quarter of the block
+        const int s = (int)(p % SUR_PTS) + ch * 8;
+        const __bf16* xr = X + (int64_t)krow * N + p / SUR_PTS * SUR_PTS + (s >> 2);
 #pragma unroll
         for (int pb = 0; pb < 4; ++pb) {
           const bf16x2 two = *(const bf16x2*)(xr + 32 * pb);
-          xv[pb] = two[0];
-          xv[4 + pb] = two[1];
+          rb[k][pb] = two[0];
+          rb[k][4 + pb] = two[1];
         }
       }
-      *(bf16x8*)(sb + so) = xv;
+    }
+  };
+  fetch(pbeg);
+  for (int64_t p = pbeg; p < pend; p += WG_PSTEP) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int q = tid + k * SUR_THREADS, row = q / (WG_PSTEP / 8), ch = q % (WG_PSTEP / 8);
+      const int so = row * WG_PSTEP + ((ch ^ (row & 7)) << 3);
+      *(bf16x8*)(sa + so) = ra[k];
+      *(bf16x8*)(sb + so) = rb[k];
     }
     __syncthreads();
+    if (p + WG_PSTEP < pend) fetch(p + WG_PSTEP);
 #pragma unroll
     for (int ks = 0; ks < WG_PSTEP / 16; ++ks) {
       const int ch = ks * 2 + half;
