@@ -673,9 +673,15 @@ int bldfm_launch_all(const PlanDev& P, const LinePlan& L, const ExecBufs& B, int
     const int rc = bldfm_launch_sur_plan(P, B, grid_cap, stream);
     if (rc) return rc;
     if (P.tot_spot > 0) {
-      k_sur_spot<true><<<grid_for(P.tot_spot, grid_cap), 256, 0, stream>>>(P, B);
+      // a launch over instances of the other rounding alone costs 4.6 us
+      bool used[2] = {false, false};  // fused, exact
+      for (int v = 0; v < 4; ++v) {
+        used[0] |= P.variant_used[v][0] != 0;
+        used[1] |= P.variant_used[v][1] || P.pair_used[v];
+      }
+      if (used[1]) k_sur_spot<true><<<grid_for(P.tot_spot, grid_cap), 256, 0, stream>>>(P, B);
       LAUNCH_CHECK();
-      k_sur_spot<false><<<grid_for(P.tot_spot, grid_cap), 256, 0, stream>>>(P, B);
+      if (used[0]) k_sur_spot<false><<<grid_for(P.tot_spot, grid_cap), 256, 0, stream>>>(P, B);
       LAUNCH_CHECK();
     }
     k_sur_gate<<<gi, 256, 0, stream>>>(P, B);
