@@ -117,28 +117,42 @@ __device__ __forceinline__ int fdiv(int j, uint64_t m) { return (int)(((uint64_t
 // of the factorisations used here.  The map only moves bits 3-5 into bits
 // 0-2, so phys(i + 64 m) = phys(i) + 64 m: an access pattern with a stride
 // that is a multiple of 64 needs one swizzle per thread, not per element.
-struct Lds {
-  double2* p;
+//
+// With C > 1 a workgroup transforms C lines that are neighbours in memory,
+// neighbouring lanes taking the same element of neighbouring lines: element i
+// of line c lives at phys(i) * C + c, and a strided gather or scatter of the
+// lines moves C * 16 consecutive bytes.
+template <int C>
+struct LdsT {
+  double2* p;  // element 0 of this lane's line
   int swz;
   __device__ __forceinline__ int phys(int i) const { return i ^ ((i >> 3) & swz); }
-  __device__ __forceinline__ double2& operator[](int i) const { return p[phys(i)]; }
+  __device__ __forceinline__ double2& raw(int ph) const { return p[ph * C]; }
+  __device__ __forceinline__ double2& operator[](int i) const { return raw(phys(i)); }
 };
-__device__ __forceinline__ Lds lds_view(double2* p, int n) { return Lds{p, (n & 7) ? 0 : 7}; }
+typedef LdsT<1> Lds;
+template <int C = 1>
+__device__ __forceinline__ LdsT<C> lds_view(double2* p, int n) { return LdsT<C>{p, (n & 7) ? 0 : 7}; }
 
 // Source and sink of the intermediate stages: the LDS buffer.
+template <int C>
 struct LdsIn {
-  Lds b;
+  LdsT<C> b;
   __device__ __forceinline__ double2 operator()(int i) const { return b[i]; }
 };
+template <int C>
 struct LdsOut {
-  Lds b;
+  LdsT<C> b;
   __device__ __forceinline__ void operator()(int i, double2 v) const { b[i] = v; }
 };
+template <class A> struct is_lds { static constexpr bool value = false; };
+template <int C> struct is_lds<LdsIn<C>> { static constexpr bool value = true; };
+template <int C> struct is_lds<LdsOut<C>> { static constexpr bool value = true; };
 
 // Twiddles W_n^t from two short tables in LDS: with t = hi*L + lo (L = 2^lb,
 // L*L >= n), W^t = W^{hi*L} * W^{lo}.  Both factors are correctly rounded
 // table entries, so W^t is within a few ulp; the tables (L + ceil(n/L)
-// entries, 88 for n = 1536) sit behind the transform buffer and replace a
+// entries, 88 for n = 1536) sit behind the transform buffers and replace a
 // dependent global load per stage by two LDS reads (tw_split_log2 and
 // tw_table_len live with the plan types).
 struct TwLds {
@@ -151,14 +165,12 @@ struct TwLds {
 };
 // Fill the tables at dst from the n-entry global table; the caller
 // synchronises the workgroup before the first lookup.
-__device__ __forceinline__ TwLds tw_tables(double2* dst, const double2* __restrict__ tw, int n, int tid, int T) {
+__device__ __forceinline__ TwLds tw_tables(double2* dst, const double2* __restrict__ tw, int n) {
+  const int tid = (int)threadIdx.x, T = (int)blockDim.x;
   const int lb = tw_split_log2(n), L = 1 << lb, nhi = (n + L - 1) >> lb;
   for (int i = tid; i < L + nhi; i += T) dst[i] = i < L ? tw[i < n ? i : 0] : tw[(i - L) << lb];
   return TwLds{dst, dst + L, lb};
 }
-
-template <class A, class B> struct same_t { static constexpr bool value = false; };
-template <class A> struct same_t<A, A> { static constexpr bool value = true; };
 
 // Stage constants: radix R, Ns, twiddle index step n/(Ns*R), and the
 // multiply-high divisor of Ns (unused in the first stage, where Ns = 1).
@@ -175,18 +187,18 @@ struct StageK {
 template <int R, int MAXB, bool INV, bool FIRST, class In, class Out>
 __device__ __forceinline__ void stage_r(In in, Out out, int n, StageK K, TwLds tw,
                                         int tid, int T) {
-  constexpr bool to_lds = same_t<Out, LdsOut>::value;
+  constexpr bool to_lds = is_lds<Out>::value;
   const int nb = n / R;
   double2 x[MAXB][R];
 #pragma unroll
   for (int b = 0; b < MAXB; ++b) {
     const int j = tid + b * T;
     if (j < nb) {
-      if constexpr (same_t<In, LdsIn>::value) {
+      if constexpr (is_lds<In>::value) {
         if ((nb & 63) == 0) {  // phys(j + r*nb) = phys(j) + r*nb
           const int pj = in.b.phys(j);
 #pragma unroll
-          for (int r = 0; r < R; ++r) x[b][r] = in.b.p[pj + r * nb];
+          for (int r = 0; r < R; ++r) x[b][r] = in.b.raw(pj + r * nb);
         } else {
 #pragma unroll
           for (int r = 0; r < R; ++r) x[b][r] = in(j + r * nb);
@@ -225,16 +237,16 @@ __device__ __forceinline__ void stage_r(In in, Out out, int n, StageK K, TwLds t
         const int q = (int)__umulhi((unsigned)j, K.magic);
         base = q * K.Ns * (R - 1) + j;  // q*Ns*R + k with k = j - q*Ns
       }
-      if constexpr (same_t<Out, LdsOut>::value) {
-        const Lds& L = out.b;
+      if constexpr (is_lds<Out>::value) {
+        const auto& L = out.b;
         if (FIRST && R == 8) {  // element 8j + r: bits 3-5 are j & 7
           const int jm = j & L.swz;
 #pragma unroll
-          for (int r = 0; r < R; ++r) L.p[base + (r ^ jm)] = x[b][r];
+          for (int r = 0; r < R; ++r) L.raw(base + (r ^ jm)) = x[b][r];
         } else if (!FIRST && (K.Ns & 63) == 0) {
           const int pb = L.phys(base);
 #pragma unroll
-          for (int r = 0; r < R; ++r) L.p[pb + r * K.Ns] = x[b][r];
+          for (int r = 0; r < R; ++r) L.raw(pb + r * K.Ns) = x[b][r];
         } else {
 #pragma unroll
           for (int r = 0; r < R; ++r) L[base + r * (FIRST ? 1 : K.Ns)] = x[b][r];
@@ -252,7 +264,7 @@ __device__ __forceinline__ void stage_r(In in, Out out, int n, StageK K, TwLds t
 template <int MAXE, bool INV, bool FIRST, class In, class Out>
 __device__ __forceinline__ void stage_generic(In in, Out out, int n, int R, StageK K,
                                               TwLds tw, int tid, int T) {
-  constexpr bool to_lds = same_t<Out, LdsOut>::value;
+  constexpr bool to_lds = is_lds<Out>::value;
   const int nb = n / R;
   const int Ns = FIRST ? 1 : K.Ns;
   const uint64_t mR = div_magic(R);
@@ -312,9 +324,11 @@ __device__ __forceinline__ void run_stage(int R, In in, Out out, int n, StageK K
 // the tables, so the workgroup synchronises before refilling them); the
 // transform buffer itself needs no such care, since every stage that writes
 // buf synchronises the workgroup before its scatter.
-template <int MAXE, bool INV, class In, class Out>
-__device__ __forceinline__ void lds_fft(Lds buf, const FftPlan* Pg, const double2* __restrict__ twg, int tid0,
-                                        int T0, In in, Out out, bool reuse) {
+// tid0, T0: this lane's index and the lanes of its line (the whole workgroup
+// for C = 1); twbuf: the tables' place, behind the C buffers.
+template <int MAXE, bool INV, int C, class In, class Out>
+__device__ __forceinline__ void lds_fft(LdsT<C> buf, double2* twbuf, const FftPlan* Pg,
+                                        const double2* __restrict__ twg, int tid0, int T0, In in, Out out, bool reuse) {
   typedef const __attribute__((address_space(4))) FftPlan cplan;
   const cplan& P = *(const cplan*)Pg;
   const int n = P.n;
@@ -324,13 +338,13 @@ __device__ __forceinline__ void lds_fft(Lds buf, const FftPlan* Pg, const double
     return;
   }
   if (reuse) __syncthreads();
-  const TwLds tw = tw_tables(buf.p + n, twg, n, tid0, T0);
+  const TwLds tw = tw_tables(twbuf, twg, n);
   {  // the radix-2/3/4/5/8 first stage reads no twiddle before its barrier
     const int R0 = P.radix[0];
     if (R0 != 2 && R0 != 3 && R0 != 4 && R0 != 5 && R0 != 8) __syncthreads();
   }
-  const LdsIn li{buf};
-  const LdsOut lo{buf};
+  const LdsIn<C> li{buf};
+  const LdsOut<C> lo{buf};
   // Each stage takes opaque copies of tid and T: without them the compiler
   // hoists every stage variant's index arithmetic out of the stage loop and
   // keeps it live across all of them (doubling the VGPR count).

@@ -20,8 +20,8 @@ template <int MAXE>
 __device__ __forceinline__ void fft_plain(bool inv, const FftPlan* F, int n, const double2* __restrict__ tw, int tid,
                                           int T, StridedIn in, StridedOut out, bool reuse) {
   const bldfm_fft::Lds buf = bldfm_fft::lds_view(smem, n);
-  if (inv) bldfm_fft::lds_fft<MAXE, true>(buf, F, tw, tid, T, in, out, reuse);
-  else bldfm_fft::lds_fft<MAXE, false>(buf, F, tw, tid, T, in, out, reuse);
+  if (inv) bldfm_fft::lds_fft<MAXE, true>(buf, smem + n, F, tw, tid, T, in, out, reuse);
+  else bldfm_fft::lds_fft<MAXE, false>(buf, smem + n, F, tw, tid, T, in, out, reuse);
 }
 
 template <int MAXE, int MAXT>
@@ -51,6 +51,47 @@ __global__ __launch_bounds__(MAXT) void k_fft2_cols(const FftPlan* F, const doub
   }
 }
 
+// C neighbouring columns per workgroup (ncols rounded up to tiles of C within
+// an array): neighbouring lanes hold neighbouring columns, so loads and stores
+// move C * 16 consecutive bytes.  One column per workgroup wrote 2.6 times the
+// result's bytes (16-byte pieces of lines that left the L2 before the seven
+// other columns came).  2 x 2048^2, both passes: 212 -> 134 us; 4 x 1024^2: 156 -> 70.
+template <int C>
+struct TileIn {
+  const double2* __restrict__ src;
+  int64_t stride;
+  bool live;
+  __device__ __forceinline__ double2 operator()(int i) const { return live ? src[(int64_t)i * stride] : cmk(0.0, 0.0); }
+};
+struct TileOut {
+  double2* __restrict__ dst;
+  int64_t stride;
+  double scale;
+  bool live;
+  __device__ __forceinline__ void operator()(int o, double2 v) const {
+    if (live) dst[(int64_t)o * stride] = cscale(scale, v);
+  }
+};
+template <int C>
+__global__ __launch_bounds__(1024) void k_fft2_col_tiles(const FftPlan* F, const double2* __restrict__ tw,
+                                                       const double2* __restrict__ mid, double2* __restrict__ out,
+                                                       int32_t n0, int32_t n1, int64_t ntiles, double scale, bool inv) {
+  const int c = (int)threadIdx.x % C, t = (int)threadIdx.x / C, T = (int)blockDim.x / C;
+  const int per = (n1 + C - 1) / C;
+  for (int64_t w = blockIdx.x; w < ntiles; w += gridDim.x) {
+    const int64_t tile = gridDim.x >= ntiles ? xcd_swizzle(w, ntiles) : w;
+    const int64_t b = tile / per;
+    const int col = (int)(tile % per) * C + c;
+    const int64_t o = b * (int64_t)n0 * n1 + col;
+    const bool live = col < n1;
+    const bldfm_fft::LdsT<C> buf = bldfm_fft::lds_view<C>(smem + c, n0);
+    const TileIn<C> in{mid + o, n1, live};
+    const TileOut dst{out + o, n1, scale, live};
+    if (inv) bldfm_fft::lds_fft<FFT_SMALL_E, true>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
+    else bldfm_fft::lds_fft<FFT_SMALL_E, false>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
+  }
+}
+
 // Split (four-step) lines of the plain 2-D FFT: `rows` selects the rows of
 // the (n0, n1) arrays (line r at r*n1, stride 1), else their columns (line c
 // at (c / n1)*n0*n1 + c % n1, stride n1); scr holds nlines x n values.
@@ -71,15 +112,28 @@ __global__ __launch_bounds__(MAXT) void k_fft2_long(FftSplit S, const double2* _
     if constexpr (!STEPB) {
       const SubIn<StridedIn> src{StridedIn{in + base, stride}, s2, sub};
       const TwiddleOut dst{sc + (int64_t)sub * s1, S.tw, sub, inv};
-      if (inv) bldfm_fft::lds_fft<MAXE, true>(buf0, S.F1, S.tw1, tid, T, src, dst, b != blockIdx.x);
-      else bldfm_fft::lds_fft<MAXE, false>(buf0, S.F1, S.tw1, tid, T, src, dst, b != blockIdx.x);
+      if (inv) bldfm_fft::lds_fft<MAXE, true>(buf0, smem + (STEPB ? s2 : s1), S.F1, S.tw1, tid, T, src, dst, b != blockIdx.x);
+      else bldfm_fft::lds_fft<MAXE, false>(buf0, smem + (STEPB ? s2 : s1), S.F1, S.tw1, tid, T, src, dst, b != blockIdx.x);
     } else {
       const ScrIn src{sc + sub, s1};
       const SubOut<StridedOut> dst{StridedOut{out + base, stride, scale}, s1, sub};
-      if (inv) bldfm_fft::lds_fft<MAXE, true>(buf0, S.F2, S.tw2, tid, T, src, dst, b != blockIdx.x);
-      else bldfm_fft::lds_fft<MAXE, false>(buf0, S.F2, S.tw2, tid, T, src, dst, b != blockIdx.x);
+      if (inv) bldfm_fft::lds_fft<MAXE, true>(buf0, smem + (STEPB ? s2 : s1), S.F2, S.tw2, tid, T, src, dst, b != blockIdx.x);
+      else bldfm_fft::lds_fft<MAXE, false>(buf0, smem + (STEPB ? s2 : s1), S.F2, S.tw2, tid, T, src, dst, b != blockIdx.x);
     }
   }
+}
+
+// Columns per workgroup of the column pass: as many as 1024 threads of eight
+// values hold (their buffers are then 128 KB), up to a cache line; one where all
+// columns together are fewer than the CUs (48 x 64: 4.5 us against 5.6 in tiles
+// of eight; 512 x 512: 11.5 against 7.3) and where a prime factor above 5 makes
+// the arithmetic the bound (1001 x 1386: 325 us against 357, both passes and the
+// conversions); 0: the kernel of long columns.
+static int fft2_tile(int n0, int64_t ncols) {
+  int m = n0;
+  for (const int p : {2, 3, 5})
+    while (m % p == 0) m /= p;
+  return n0 > 2048 ? 0 : ncols < 256 || m > 1 ? 1 : n0 <= 1024 ? 8 : 4;
 }
 
 int bldfm_launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, int32_t batch,
@@ -127,8 +181,15 @@ int bldfm_launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_
       LAUNCH_CHECK();
       k_fft2_long<BLDFM_FFT_MAXE, 1024, true><<<gb, threads, lds_bytes, stream>>>(A0, nullptr, out, scr, 0, n0, n1, ncols, scale, inv);
     }
-  } else if (small) {
-    k_fft2_cols<FFT_SMALL_E, 256><<<grid_for(ncols, grid_cap), threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
+  } else if (fft2_tile(n0, ncols)) {
+    const int c = fft2_tile(n0, ncols);
+    const int64_t tiles = (int64_t)batch * ((n1 + c - 1) / c);
+    const int t = (n0 + FFT_SMALL_E - 1) / FFT_SMALL_E;                     // lanes of a column
+    const unsigned nt = (unsigned)((t * c + 63) / 64 * 64);
+    const size_t lds = ((size_t)n0 * c + tw_table_len(n0)) * 16;
+    if (c == 8) k_fft2_col_tiles<8><<<grid_for(tiles, grid_cap), nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
+    else if (c == 1) k_fft2_col_tiles<1><<<grid_for(tiles, grid_cap), nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
+    else k_fft2_col_tiles<4><<<grid_for(tiles, grid_cap), nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
   } else {
     k_fft2_cols<BLDFM_FFT_MAXE, 1024><<<grid_for(ncols, grid_cap), threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
   }
@@ -138,9 +199,12 @@ int bldfm_launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_
 
 void bldfm_fft2_lds_attr(int bytes) {
   const void* fns[] = {
-      (const void*)k_fft2_rows<FFT_SMALL_E, 256>, (const void*)k_fft2_cols<FFT_SMALL_E, 256>,
+      (const void*)k_fft2_rows<FFT_SMALL_E, 256>,
       (const void*)k_fft2_long<FFT_SMALL_E, 256, false>, (const void*)k_fft2_long<FFT_SMALL_E, 256, true>,
       (const void*)k_fft2_rows<BLDFM_FFT_MAXE, 1024>, (const void*)k_fft2_cols<BLDFM_FFT_MAXE, 1024>,
       (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, false>, (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, true>};
   for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  const int tile = (2048 * 4 + tw_table_len(2048)) * 16;
+  const void* tiled[] = {(const void*)k_fft2_col_tiles<1>, (const void*)k_fft2_col_tiles<4>, (const void*)k_fft2_col_tiles<8>};
+  for (const void* f : tiled) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, tile);
 }

@@ -90,8 +90,8 @@ template <int MAXE, class In, class Out>
 __device__ __forceinline__ void fft_dir(bool inv, const cplan_t& F, const double2* __restrict__ tw, int tid, int T,
                                         In in, Out out, bool reuse) {
   const bldfm_fft::Lds buf = bldfm_fft::lds_view(smem, F.n);
-  if (inv) bldfm_fft::lds_fft<MAXE, true>(buf, (const FftPlan*)&F, tw + F.tw_off, tid, T, in, out, reuse);
-  else bldfm_fft::lds_fft<MAXE, false>(buf, (const FftPlan*)&F, tw + F.tw_off, tid, T, in, out, reuse);
+  if (inv) bldfm_fft::lds_fft<MAXE, true>(buf, smem + F.n, (const FftPlan*)&F, tw + F.tw_off, tid, T, in, out, reuse);
+  else bldfm_fft::lds_fft<MAXE, false>(buf, smem + F.n, (const FftPlan*)&F, tw + F.tw_off, tid, T, in, out, reuse);
 }
 
 // The four passes, each as a factory of (plan, source, sink, direction) for
