@@ -103,6 +103,58 @@ __device__ __forceinline__ void butterfly<8>(double2* x, bool inv) {
   x[7] = csub(e[3], o3);
 }
 
+// Cosines and sines of 2 pi j/P, j = 1 .. (P-1)/2, of the prime butterflies.
+template <int P> struct PrimeRoots;
+template <> struct PrimeRoots<7> {
+  static constexpr double c[3] = {0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624};
+  static constexpr double s[3] = {0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
+};
+template <> struct PrimeRoots<11> {
+  static constexpr double c[5] = {0.84125353283118116886, 0.41541501300188642553, -0.14231483827328514044,
+                                  -0.65486073394528506406, -0.95949297361449738989};
+  static constexpr double s[5] = {0.54064081745559758211, 0.90963199535451837141, 0.98982144188093273238,
+                                  0.75574957435425828378, 0.28173255684142969772};
+};
+template <> struct PrimeRoots<13> {
+  static constexpr double c[6] = {0.88545602565320989590, 0.56806474673115580251, 0.12053668025532305335,
+                                  -0.35460488704253562597, -0.74851074817110109863, -0.97094181742605202716};
+  static constexpr double s[6] = {0.46472317204376854566, 0.82298386589365639458, 0.99270887409805399281,
+                                  0.93501624268541482344, 0.66312265824079520238, 0.23931566428755776715};
+};
+
+// Length-P DFT of an odd prime P from the sums and differences of the pairs
+// (k, P - k): (P-1)^2 real products instead of the generic stage's P twiddled
+// complex ones per output.
+template <int P>
+__device__ __forceinline__ void butterfly_prime(double2* x, bool inv) {
+  constexpr int H = (P - 1) / 2;
+  double2 t[H], d[H], y0 = x[0];
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    t[k] = cadd(x[k + 1], x[P - 1 - k]);
+    d[k] = csub(x[k + 1], x[P - 1 - k]);
+    y0 = cadd(y0, t[k]);
+  }
+#pragma unroll
+  for (int m = 1; m <= H; ++m) {
+    double2 a = x[0], b = cmk(0.0, 0.0);
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+      const int j = m * k % P, q = j <= H ? j : P - j;
+      const double c = PrimeRoots<P>::c[q - 1], s = j <= H ? PrimeRoots<P>::s[q - 1] : -PrimeRoots<P>::s[q - 1];
+      a = cmk(fma(c, t[k - 1].x, a.x), fma(c, t[k - 1].y, a.y));
+      b = cmk(fma(s, d[k - 1].x, b.x), fma(s, d[k - 1].y, b.y));
+    }
+    b = mul_si(b, inv);
+    x[m] = cadd(a, b);  // x[m] and x[P - m] are read again only through t and d
+    x[P - m] = csub(a, b);
+  }
+  x[0] = y0;
+}
+template <> __device__ __forceinline__ void butterfly<7>(double2* x, bool inv) { butterfly_prime<7>(x, inv); }
+template <> __device__ __forceinline__ void butterfly<11>(double2* x, bool inv) { butterfly_prime<11>(x, inv); }
+template <> __device__ __forceinline__ void butterfly<13>(double2* x, bool inv) { butterfly_prime<13>(x, inv); }
+
 // j / d for 0 <= j, d < 2^16 by multiply-high: with m = floor(2^32/d) + 1 the
 // error of j*m/2^32 against j/d is below 2^-16 < 1/d, so the floor is exact.
 __device__ __forceinline__ uint64_t div_magic(int d) { return (1ull << 32) / (uint64_t)d + 1ull; }
@@ -300,7 +352,9 @@ __device__ __forceinline__ void stage_generic(In in, Out out, int n, int R, Stag
   if (to_lds) __syncthreads();
 }
 
-template <int MAXE, bool INV, bool FIRST, class In, class Out>
+// PRIMES: with the butterflies of 7, 11 and 13 (their registers would cost the
+// solver's passes, whose rough lengths run as chirps, a wave a SIMD).
+template <int MAXE, bool INV, bool FIRST, bool PRIMES, class In, class Out>
 __device__ __forceinline__ void run_stage(int R, In in, Out out, int n, StageK K, TwLds tw,
                                           int tid, int T) {
   switch (R) {
@@ -309,7 +363,14 @@ __device__ __forceinline__ void run_stage(int R, In in, Out out, int n, StageK K
     case 4: stage_r<4, (MAXE + 3) / 4, INV, FIRST>(in, out, n, K, tw, tid, T); break;
     case 5: stage_r<5, (MAXE + 4) / 5, INV, FIRST>(in, out, n, K, tw, tid, T); break;
     case 8: stage_r<8, (MAXE + 7) / 8, INV, FIRST>(in, out, n, K, tw, tid, T); break;
-    default: stage_generic<MAXE, INV, FIRST>(in, out, n, R, K, tw, tid, T); break;
+    default:
+      if constexpr (PRIMES) {
+        if (R == 7) return stage_r<7, (MAXE + 6) / 7, INV, FIRST>(in, out, n, K, tw, tid, T);
+        if (R == 11) return stage_r<11, (MAXE + 10) / 11, INV, FIRST>(in, out, n, K, tw, tid, T);
+        if (R == 13) return stage_r<13, (MAXE + 12) / 13, INV, FIRST>(in, out, n, K, tw, tid, T);
+      }
+      stage_generic<MAXE, INV, FIRST>(in, out, n, R, K, tw, tid, T);
+      break;
   }
 }
 
@@ -326,7 +387,7 @@ __device__ __forceinline__ void run_stage(int R, In in, Out out, int n, StageK K
 // buf synchronises the workgroup before its scatter.
 // tid0, T0: this lane's index and the lanes of its line (the whole workgroup
 // for C = 1); twbuf: the tables' place, behind the C buffers.
-template <int MAXE, bool INV, int C, class In, class Out>
+template <int MAXE, bool INV, bool PRIMES = false, int C, class In, class Out>
 __device__ __forceinline__ void lds_fft(LdsT<C> buf, double2* twbuf, const FftPlan* Pg,
                                         const double2* __restrict__ twg, int tid0, int T0, In in, Out out, bool reuse) {
   typedef const __attribute__((address_space(4))) FftPlan cplan;
@@ -353,10 +414,10 @@ __device__ __forceinline__ void lds_fft(LdsT<C> buf, double2* twbuf, const FftPl
     int tid = tid0, T = T0;
     asm volatile("" : "+v"(tid), "+s"(T));
     if (nstage == 1) {
-      run_stage<MAXE, INV, true>(P.radix[0], in, out, n, K0, tw, tid, T);
+      run_stage<MAXE, INV, true, PRIMES>(P.radix[0], in, out, n, K0, tw, tid, T);
       return;
     }
-    run_stage<MAXE, INV, true>(P.radix[0], in, lo, n, K0, tw, tid, T);
+    run_stage<MAXE, INV, true, PRIMES>(P.radix[0], in, lo, n, K0, tw, tid, T);
   }
   int Ns = P.radix[0];
   for (int s = 1; s < nstage; ++s) {
@@ -364,8 +425,8 @@ __device__ __forceinline__ void lds_fft(LdsT<C> buf, double2* twbuf, const FftPl
     const StageK K{Ns, P.stride[s], P.magic[s]};
     int tid = tid0, T = T0;
     asm volatile("" : "+v"(tid), "+s"(T));
-    if (s == nstage - 1) run_stage<MAXE, INV, false>(R, li, out, n, K, tw, tid, T);
-    else run_stage<MAXE, INV, false>(R, li, lo, n, K, tw, tid, T);
+    if (s == nstage - 1) run_stage<MAXE, INV, false, PRIMES>(R, li, out, n, K, tw, tid, T);
+    else run_stage<MAXE, INV, false, PRIMES>(R, li, lo, n, K, tw, tid, T);
     Ns *= R;
   }
 }

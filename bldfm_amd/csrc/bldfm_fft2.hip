@@ -20,8 +20,8 @@ template <int MAXE>
 __device__ __forceinline__ void fft_plain(bool inv, const FftPlan* F, int n, const double2* __restrict__ tw, int tid,
                                           int T, StridedIn in, StridedOut out, bool reuse) {
   const bldfm_fft::Lds buf = bldfm_fft::lds_view(smem, n);
-  if (inv) bldfm_fft::lds_fft<MAXE, true>(buf, smem + n, F, tw, tid, T, in, out, reuse);
-  else bldfm_fft::lds_fft<MAXE, false>(buf, smem + n, F, tw, tid, T, in, out, reuse);
+  if (inv) bldfm_fft::lds_fft<MAXE, true, true>(buf, smem + n, F, tw, tid, T, in, out, reuse);
+  else bldfm_fft::lds_fft<MAXE, false, true>(buf, smem + n, F, tw, tid, T, in, out, reuse);
 }
 
 template <int MAXE, int MAXT>
@@ -42,7 +42,8 @@ __global__ __launch_bounds__(MAXT) void k_fft2_cols(const FftPlan* F, const doub
   for (int64_t w = blockIdx.x; w < ncols; w += gridDim.x) {
     // eight neighbouring columns share every 128-byte line: each XCD takes a
     // contiguous range of them, so a line is fetched into one L2 and not into
-    // eight (both passes of 2 x 2048^2 complex128: 302 -> 212 us)
+    // eight (both passes of 2 x 2048^2 complex128, before its
+    // columns ran in tiles: 302 -> 212 us)
     const int64_t c = gridDim.x >= ncols ? xcd_swizzle(w, ncols) : w;
     const int64_t b = c / n1, col = c % n1;
     const int64_t o = b * (int64_t)n0 * n1 + col;
@@ -87,8 +88,8 @@ __global__ __launch_bounds__(1024) void k_fft2_col_tiles(const FftPlan* F, const
     const bldfm_fft::LdsT<C> buf = bldfm_fft::lds_view<C>(smem + c, n0);
     const TileIn<C> in{mid + o, n1, live};
     const TileOut dst{out + o, n1, scale, live};
-    if (inv) bldfm_fft::lds_fft<FFT_SMALL_E, true>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
-    else bldfm_fft::lds_fft<FFT_SMALL_E, false>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
+    if (inv) bldfm_fft::lds_fft<FFT_SMALL_E, true, true>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
+    else bldfm_fft::lds_fft<FFT_SMALL_E, false, true>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
   }
 }
 
@@ -126,12 +127,14 @@ __global__ __launch_bounds__(MAXT) void k_fft2_long(FftSplit S, const double2* _
 // Columns per workgroup of the column pass: as many as 1024 threads of eight
 // values hold (their buffers are then 128 KB), up to a cache line; one where all
 // columns together are fewer than the CUs (48 x 64: 4.5 us against 5.6 in tiles
-// of eight; 512 x 512: 11.5 against 7.3) and where a prime factor above 5 makes
-// the arithmetic the bound (1001 x 1386: 325 us against 357, both passes and the
-// conversions); 0: the kernel of long columns.
+// of eight; 512 x 512: 11.5 against 7.3) and where a prime factor above 13 takes
+// the generic stage, which is arithmetic bound and runs best over many small
+// workgroups (with 7, 11 and 13 in the generic stage too, 1001 x 1386 x 4 took
+// 250 us in tiles of one and 282 of eight; with their butterflies 119 and 104);
+// 0: the kernel of long columns.
 static int fft2_tile(int n0, int64_t ncols) {
   int m = n0;
-  for (const int p : {2, 3, 5})
+  for (const int p : {2, 3, 5, 7, 11, 13})
     while (m % p == 0) m /= p;
   return n0 > 2048 ? 0 : ncols < 256 || m > 1 ? 1 : n0 <= 1024 ? 8 : 4;
 }

@@ -21,3 +21,17 @@ def test_column_tiles_match_numpy(n0, n1, batch):
     x = rng.standard_normal((batch, n0, n1)) + 1j * rng.standard_normal((batch, n0, n1))
     for got, want in ((fft_manager.fft2(x), np.fft.fft2(x)), (fft_manager.ifft2(x, norm="ortho"), np.fft.ifft2(x, norm="ortho"))):
         assert np.linalg.norm(got - want) <= 4e-15 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("n0,n1", [
+    (7, 11), (13, 49), (121, 169), (343, 77), (91, 1001), (1386, 143), (2197, 14), (22, 2401), (26, 7007), (7007, 3),
+    (28, 1331), (17, 1309), (4, 15015), (15015, 2)])
+def test_prime_butterflies_match_numpy(n0, n1):
+    """Radices 7, 11 and 13 alone, repeated, mixed with each other and with the
+    generic stage (17), in rows, columns, both register sizes and split lines."""
+    from bldfm_amd import fft_manager
+
+    rng = np.random.default_rng(n0 * 3 + n1)
+    x = rng.standard_normal((n0, n1)) + 1j * rng.standard_normal((n0, n1))
+    for got, want in ((fft_manager.fft2(x), np.fft.fft2(x)), (fft_manager.ifft2(x, norm="ortho"), np.fft.ifft2(x, norm="ortho"))):
+        assert np.linalg.norm(got - want) <= 4e-15 * np.linalg.norm(want)
