@@ -131,6 +131,7 @@ SIGNATURES = {
     "bldfm_math_probe": (ctypes.c_int, [_I32, _P, _P, _I64, _P, _P]),
     "bldfm_fft2_workspace_bytes": (ctypes.c_size_t, [_I32, _I32, _I32]),
     "bldfm_fft2": (ctypes.c_int, [ctypes.c_int, _I32, _I32, _I32, _P, _P, _I32, _D, _P, _P]),
+    "bldfm_fft2_c64": (ctypes.c_int, [ctypes.c_int, _I32, _I32, _I32, _P, _P, _I32, _D, _P, _P]),
     "bldfm_sur_sizes": (ctypes.c_int, [ctypes.POINTER(_I64), ctypes.POINTER(_I64), ctypes.POINTER(_I64), ctypes.POINTER(_I32)]),
     "bldfm_sur_met": (ctypes.c_int, [ctypes.POINTER(Met), _I32, _P]),
     "bldfm_transfer_tables": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(Met), _I32, _I32, _P, _P, _P]),

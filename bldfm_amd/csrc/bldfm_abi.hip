@@ -1067,8 +1067,8 @@ size_t bldfm_fft2_workspace_bytes(int32_t n0, int32_t n1, int32_t batch) {
   return (size_t)n0 * n1 * batch * sizeof(double2) * (split ? 2 : 1);
 }
 
-int bldfm_fft2(int device, int32_t n0, int32_t n1, int32_t batch, const double* in, double* out,
-               int32_t sign, double scale, void* workspace, hipStream_t stream) {
+static int fft2_impl(int device, int32_t n0, int32_t n1, int32_t batch, bool single, const void* in, void* out,
+                     int32_t sign, double scale, void* workspace, hipStream_t stream) {
   if (n0 <= 0 || n1 <= 0 || batch <= 0 || !in || !out || !workspace)
     return fail(BLDFM_EINVAL, "bad fft2 arguments");
   if (sign != 1 && sign != -1) return fail(BLDFM_EINVAL, "sign must be +1 or -1");
@@ -1104,11 +1104,21 @@ int bldfm_fft2(int device, int32_t n0, int32_t n1, int32_t batch, const double* 
   set_lds_attr(fft_lds_bytes(nmax));
   double2* mid = (double2*)workspace;
   double2* scr = (s0 || s1) ? mid + (int64_t)n0 * n1 * batch : nullptr;
-  rc = bldfm_launch_fft2(A[0], n0, A[1], n1, batch, (const double2*)in, mid, scr, (double2*)out, sign, scale,
-                         fft_threads_for(nmax), fft_lds_bytes(nmax), kGridCap, stream);
+  rc = bldfm_launch_fft2(A[0], n0, A[1], n1, batch, single, in, mid, scr, out, sign, scale, fft_threads_for(nmax),
+                         fft_lds_bytes(nmax), kGridCap, stream);
   if (rc) return fail(BLDFM_EHIP, std::string("fft2 launch failed: ") +
                                       hipGetErrorString((hipError_t)(-(rc + 1000))));
   return 0;
+}
+
+int bldfm_fft2(int device, int32_t n0, int32_t n1, int32_t batch, const double* in, double* out,
+               int32_t sign, double scale, void* workspace, hipStream_t stream) {
+  return fft2_impl(device, n0, n1, batch, false, in, out, sign, scale, workspace, stream);
+}
+
+int bldfm_fft2_c64(int device, int32_t n0, int32_t n1, int32_t batch, const float* in, float* out,
+                   int32_t sign, double scale, void* workspace, hipStream_t stream) {
+  return fft2_impl(device, n0, n1, batch, true, in, out, sign, scale, workspace, stream);
 }
 
 // ------------------------------------------------------------------ surrogate

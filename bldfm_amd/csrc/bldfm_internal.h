@@ -141,9 +141,10 @@ struct FftSplit {
   int32_t n1, n2;
 };
 // A0/A1: the axis lengths n0 (columns) and n1 (rows); scr: batch*n0*n1
-// values of four-step scratch when an axis is split (else unused)
-int bldfm_launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, int32_t batch,
-                      const double2* in, double2* mid, double2* scr, double2* out, int32_t sign, double scale,
+// values of four-step scratch when an axis is split (else unused); single:
+// in/out hold float2, else double2
+int bldfm_launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, int32_t batch, bool single,
+                      const void* in, double2* mid, double2* scr, void* out, int32_t sign, double scale,
                       int threads, int lds_bytes, int grid_cap, hipStream_t stream);
 void bldfm_set_fft_lds_attr(int bytes);
 void bldfm_set_line_lds_attr(int bytes);

@@ -36,10 +36,11 @@ def _fft2(x, norm, forward):
         xa = np.asarray(x)
         single = xa.dtype in (np.complex64, np.float32)
         dev = _lib.device()
-        t = torch.as_tensor(np.ascontiguousarray(xa, dtype=np.complex128), device=dev)
+        t = torch.as_tensor(np.ascontiguousarray(xa, dtype=np.complex64 if single else np.complex128), device=dev)
     else:
         single = x.dtype in (torch.complex64, torch.float32)
-        t = x.to(torch.complex128).contiguous()
+        # a lazy conjugate or negation is resolved by a converting copy only
+        t = (x.to(torch.complex64).resolve_conj().resolve_neg() if single else x.to(torch.complex128)).contiguous()
         dev = t.device
     if t.ndim < 2:
         raise ValueError("fft2 needs at least two dimensions")
@@ -49,13 +50,12 @@ def _fft2(x, norm, forward):
     if t.numel() > 0:
         ws = torch.empty(lib.bldfm_fft2_workspace_bytes(n0, n1, batch), dtype=torch.uint8, device=dev)
         sign = -1 if forward else 1
+        fft2 = lib.bldfm_fft2_c64 if single else lib.bldfm_fft2
         _lib.check(
-            lib.bldfm_fft2(dev.index, n0, n1, batch, _lib.ptr(t), _lib.ptr(out), sign,
+            fft2(dev.index, n0, n1, batch, _lib.ptr(t), _lib.ptr(out), sign,
                            _scale(norm, n0 * n1, forward), _lib.ptr(ws), _lib.stream_handle(dev)),
             "fft2",
         )
-    if single:
-        out = out.to(torch.complex64)
     return out.cpu().numpy() if as_numpy else out
 
 

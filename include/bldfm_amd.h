@@ -254,11 +254,14 @@ int bldfm_plan_timing_end(bldfm_plan* plan, double* phase_ms, int32_t* nexecs);
  * 2-D complex FFT of `batch` contiguous (n0, n1) complex128 arrays with
  * numpy semantics: sign -1 (fft2) or +1 (ifft2), every output multiplied by
  * `scale`.  Replaces FFTManager.fft2/ifft2 (src/bldfm/fft_manager.py:78-102).
- * `workspace` needs bldfm_fft2_workspace_bytes().
+ * `workspace` needs bldfm_fft2_workspace_bytes().  bldfm_fft2_c64 takes and
+ * returns complex64, computing in FP64 between the loads and the rounding.
  */
 size_t bldfm_fft2_workspace_bytes(int32_t n0, int32_t n1, int32_t batch);
 int bldfm_fft2(int device, int32_t n0, int32_t n1, int32_t batch, const double* in, double* out,
                int32_t sign, double scale, void* workspace, hipStream_t stream);
+int bldfm_fft2_c64(int device, int32_t n0, int32_t n1, int32_t batch, const float* in, float* out,
+                   int32_t sign, double scale, void* workspace, hipStream_t stream);
 
 /*
  * Diagnostics (no counterpart in the reference): evaluates the device

@@ -89,3 +89,8 @@ def test_short_profile_arrays_raise_the_references_error(short):
     with pytest.raises(IndexError) as ge:
         solver.steady_state_transport_solver(q0, z, tuple(profs), (100.0, 100.0), 8, **kw)
     assert str(ge.value) == str(oe.value)
+
+
+def test_fft2_c64_refuses_what_fft2_refuses(lib):
+    _refused(lib, lib.bldfm_fft2_c64(0, 0, 8, 1, None, None, 1, 1.0, None, None), "bad fft2 arguments")
+    _refused(lib, lib.bldfm_fft2_c64(0, 8, -1, 1, None, None, 1, 1.0, None, None), "bad fft2 arguments")

@@ -35,3 +35,30 @@ def test_prime_butterflies_match_numpy(n0, n1):
     x = rng.standard_normal((n0, n1)) + 1j * rng.standard_normal((n0, n1))
     for got, want in ((fft_manager.fft2(x), np.fft.fft2(x)), (fft_manager.ifft2(x, norm="ortho"), np.fft.ifft2(x, norm="ortho"))):
         assert np.linalg.norm(got - want) <= 4e-15 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("n0,n1", [
+    (1, 1), (7, 300), (8, 257), (1024, 263), (1025, 260), (2049, 258), (3, 2049), (15015, 3), (3, 15015), (4100, 15015 // 5)])
+def test_complex64_rounds_only_the_result(n0, n1):
+    """complex64 and float32 fields through every kernel family, contiguous or
+    not, conjugate and negated views, eight-byte aligned: the FP64 transform
+    rounded once.  A rounding is at most 2^-24 of each part, so is their L2."""
+    import torch
+    from bldfm_amd import fft_manager
+
+    rng = np.random.default_rng(n0 + 5 * n1)
+    flat = (rng.standard_normal(n0 * n1 + 1) + 1j * rng.standard_normal(n0 * n1 + 1)).astype(np.complex64)
+    x = flat[1:].reshape(n0, n1)
+    dev = torch.as_tensor(flat, device="cuda")[1:].reshape(n0, n1)
+    assert dev.data_ptr() % 16 == 8
+    turned = torch.as_tensor(np.ascontiguousarray(x.T), device="cuda").T
+    for got, base in ((fft_manager.fft2(x), x), (fft_manager.fft2(dev), x), (fft_manager.fft2(turned), x),
+                      (fft_manager.fft2(dev.conj()), x.conj()), (fft_manager.fft2(torch._neg_view(dev)), -x),
+                      (fft_manager.fft2(x.real), x.real), (fft_manager.fft2(dev.real), x.real),
+                      (fft_manager.fft2(dev.conj().imag), -x.imag)):
+        want = np.fft.fft2(base.astype(np.complex128))
+        got = got if isinstance(got, np.ndarray) else got.cpu().numpy()
+        assert got.dtype == np.complex64
+        assert np.linalg.norm(got - want) <= 6e-8 * np.linalg.norm(want)
+    got, want = fft_manager.ifft2(dev).cpu().numpy(), np.fft.ifft2(x.astype(np.complex128))
+    assert np.linalg.norm(got - want) <= 6e-8 * np.linalg.norm(want)
