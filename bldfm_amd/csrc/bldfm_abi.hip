@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -316,7 +317,18 @@ int cached_plan(int device, int n, const FftPlan** plan, const double2** tw) {
   return 0;
 }
 
-void set_lds_attr(int bytes) { bldfm_set_fft_lds_attr(bytes); }
+// Dynamic LDS beyond the default cap, for every transform kernel: the device's
+// whole LDS, set by the first plan or plain FFT on a device and not by each call
+// (some forty runtime calls: small fft2 calls back to back took 23 us, now 20).
+// A launch asks for what it needs; two first callers set the same value.
+void set_lds_attr(int device) {
+  static std::atomic<uint64_t> done{0};
+  const uint64_t bit = device >= 0 && device < 64 ? 1ull << device : 0;
+  if (done.load(std::memory_order_acquire) & bit) return;
+  bldfm_set_fft_lds_attr(max_lds_bytes(device));
+  bldfm_set_line_lds_attr(max_lds_bytes(device));
+  done.fetch_or(bit, std::memory_order_release);
+}
 
 }  // namespace
 
@@ -843,15 +855,12 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
     V.t_long[k] = (const TileRec*)(base + o_tiles[10 + k]);
     V.tot_long[k] = tiles[10 + k][ninst];
   }
-  int line_max = 0;
   for (int k = 0; k < 4; ++k)
     for (int m = 0; m < LINE_NLM; ++m) {
       P->lines.recs[k][m] = (const TileRec*)(base + o_tiles[18 + k * LINE_NLM + m]);
       P->lines.tot[k][m] = tiles[18 + k * LINE_NLM + m][ninst];
       P->lines.lds[k][m] = line_lds[k][m];
-      line_max = std::max(line_max, line_lds[k][m]);
     }
-  if (line_max) bldfm_set_line_lds_attr(line_max);
   V.tot_tr = tiles[9][ninst];
   V.shoot_block = shoot_block;
   V.xlayout = xlayout;
@@ -877,7 +886,7 @@ int bldfm_plan_create_tuned(int device, const bldfm_instance* inst, int32_t nins
   V.tot_nyq = tiles[4][ninst];
   V.tot_inv_cols = tiles[5][ninst];
   V.tot_inv_rows = tiles[6][ninst];
-  set_lds_attr(V.fft_lds_bytes);
+  set_lds_attr(device);
 
   P->tab_doubles = off_tab;
   P->ws_cplx = off_ws;
@@ -1101,7 +1110,7 @@ static int fft2_impl(int device, int32_t n0, int32_t n1, int32_t batch, bool sin
     }
   }
   const int nmax = std::max(lds_len(n0, s0), lds_len(n1, s1));
-  set_lds_attr(fft_lds_bytes(nmax));
+  set_lds_attr(device);
   double2* mid = (double2*)workspace;
   double2* scr = (s0 || s1) ? mid + (int64_t)n0 * n1 * batch : nullptr;
   rc = bldfm_launch_fft2(A[0], n0, A[1], n1, batch, single, in, mid, scr, out, sign, scale, fft_threads_for(nmax),

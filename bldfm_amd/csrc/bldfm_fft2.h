@@ -139,18 +139,19 @@ __global__ __launch_bounds__(MAXT) void k_fft2_long(FftSplit S, const E* __restr
 }
 
 // Columns per workgroup of the column pass: as many as 1024 threads of eight
-// values hold (their buffers are then 128 KB), up to a cache line; one where all
-// columns together are fewer than the CUs (48 x 64: 4.5 us against 5.6 in tiles
-// of eight; 512 x 512: 11.5 against 7.3) and where a prime factor above 13 takes
-// the generic stage, which is arithmetic bound and runs best over many small
-// workgroups (with 7, 11 and 13 in the generic stage too, 1001 x 1386 x 4 took
-// 250 us in tiles of one and 282 of eight; with their butterflies 119 and 104);
-// 0: the kernel of long columns.
+// values hold (their buffers are then 128 KB), up to a cache line; 0: a column
+// per workgroup, for columns too long for a tile, for fields of less than 1 MB
+// or 256 columns, whose tiles are fewer than the CUs (200 x 256: 10.2 us against
+// 11.2 in tiles, 256 x 256: 11.2 and 11.1, 1000 x 256: 22.5 and 19.5, 512 x 512:
+// 20.4 and 14.2), and where a prime factor above 13 takes the generic stage,
+// which is arithmetic bound and runs best over many small workgroups
+// (2 x 97 x 300: 32 us against 40 for lanes as few as a tile's).
 inline int fft2_tile(int n0, int64_t ncols) {
   int m = n0;
   for (const int p : {2, 3, 5, 7, 11, 13})
     while (m % p == 0) m /= p;
-  return n0 > 2048 ? 0 : ncols < 256 || m > 1 ? 1 : n0 <= 1024 ? 8 : 4;
+  if (n0 > 2048 || ncols < 256 || n0 * ncols < 65536 || m > 1) return 0;
+  return n0 <= 1024 ? 8 : 4;
 }
 
 template <class E>
@@ -206,8 +207,9 @@ int launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, 
     const unsigned nt = (unsigned)((t * c + 63) / 64 * 64);
     const size_t lds = ((size_t)n0 * c + tw_table_len(n0)) * 16;
     if (c == 8) k_fft2_col_tiles<8, E><<<grid_for(tiles, grid_cap), nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
-    else if (c == 1) k_fft2_col_tiles<1, E><<<grid_for(tiles, grid_cap), nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
     else k_fft2_col_tiles<4, E><<<grid_for(tiles, grid_cap), nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
+  } else if (small) {
+    k_fft2_cols<FFT_SMALL_E, 256, E><<<grid_for(ncols, grid_cap), threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
   } else {
     k_fft2_cols<BLDFM_FFT_MAXE, 1024, E><<<grid_for(ncols, grid_cap), threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
   }
@@ -221,9 +223,7 @@ void fft2_lds_attr(int bytes) {
       (const void*)k_fft2_rows<FFT_SMALL_E, 256, E>,
       (const void*)k_fft2_long<FFT_SMALL_E, 256, false, E>, (const void*)k_fft2_long<FFT_SMALL_E, 256, true, E>,
       (const void*)k_fft2_rows<BLDFM_FFT_MAXE, 1024, E>, (const void*)k_fft2_cols<BLDFM_FFT_MAXE, 1024, E>,
-      (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, false, E>, (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, true, E>};
+      (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, false, E>, (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, true, E>,
+      (const void*)k_fft2_cols<FFT_SMALL_E, 256, E>, (const void*)k_fft2_col_tiles<4, E>, (const void*)k_fft2_col_tiles<8, E>};
   for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  const int tile = (2048 * 4 + tw_table_len(2048)) * 16;
-  const void* tiled[] = {(const void*)k_fft2_col_tiles<1, E>, (const void*)k_fft2_col_tiles<4, E>, (const void*)k_fft2_col_tiles<8, E>};
-  for (const void* f : tiled) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, tile);
 }

@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n0,n1,batch", [
     (1, 300, 1), (2, 257, 1), (8, 255, 1), (8, 256, 1), (7, 85, 3), (63, 261, 1), (64, 1003, 1), (1024, 263, 1),
-    (1025, 129, 2), (2048, 258, 1), (2047, 33, 8), (2049, 258, 1), (1024, 5, 60), (360, 2, 129)])
+    (1025, 129, 2), (2048, 258, 1), (2047, 33, 8), (2049, 258, 1), (1024, 5, 60), (360, 2, 129),
+    (8, 8195, 1), (1, 300, 220), (63, 1041, 1), (256, 255, 1), (256, 256, 1), (97, 700, 1)])
 def test_column_tiles_match_numpy(n0, n1, batch):
     from bldfm_amd import fft_manager
 
