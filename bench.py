@@ -491,7 +491,7 @@ def main():
         },
         "roofline": {
             "bound": "fp64-valu",
-            "kernel": "k_shoot<1,false,true> (vertical march + shooting)",
+            "kernel": "k_shoot_pair<false,256> (vertical march + shooting, two modes a lane)",
             "achieved": round(achieved / 1e12, 3),
             "peak": PEAK_FP64 / 1e12,
             "unit": "TFLOP/s",
