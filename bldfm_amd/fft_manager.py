@@ -39,8 +39,9 @@ def _fft2(x, norm, forward):
         t = torch.as_tensor(np.ascontiguousarray(xa, dtype=np.complex64 if single else np.complex128), device=dev)
     else:
         single = x.dtype in (torch.complex64, torch.float32)
-        # a lazy conjugate or negation is resolved by a converting copy only
-        t = (x.to(torch.complex64).resolve_conj().resolve_neg() if single else x.to(torch.complex128)).contiguous()
+        # .to() keeps the lazy conjugate or negation of a tensor that has the type already, and
+        # the kernels read the memory behind it
+        t = x.to(torch.complex64 if single else torch.complex128).resolve_conj().resolve_neg().contiguous()
         dev = t.device
     if t.ndim < 2:
         raise ValueError("fft2 needs at least two dimensions")
