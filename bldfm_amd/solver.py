@@ -201,7 +201,7 @@ def solve_device(
     src = None
     if not footprint:
         src = srf_flx if torch.is_tensor(srf_flx) else torch.as_tensor(np.ascontiguousarray(srf_flx, dtype=np.float64))
-        src = src.to(device=dev, dtype=torch.float64).contiguous()
+        src = src.to(device=dev, dtype=torch.float64).resolve_neg().contiguous()  # the kernels read memory
     odt = torch.float32 if g["out_f32"] else torch.float64
     conc = torch.empty((nslot, g["nyo"], g["nxo"]), dtype=odt, device=dev)
     flx = torch.empty_like(conc)

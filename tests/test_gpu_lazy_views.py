@@ -25,3 +25,18 @@ def test_fft_of_lazy_double_views(n0, n1):
             assert got.dtype == torch.complex128
             assert np.linalg.norm(got.cpu().numpy() - want) <= 4e-15 * np.linalg.norm(want)
     assert torch.equal(dev, before)
+
+
+def test_solve_of_a_negated_source():
+    import torch
+    from bldfm_amd import solver
+    from oracle import pbl as opbl
+
+    z, prof = opbl.vertical_profiles(8, 10.0, (3.0, 1.5), ustar=0.4, mol=-60.0)
+    q = torch.as_tensor(np.random.default_rng(2).random((40, 48)), device="cuda")
+    kw = dict(modes=(48, 40), halo=100.0, precision="double")
+    got = solver.solve_device(torch._neg_view(q), z, prof, (480.0, 400.0), [2, 8], **kw)
+    want = solver.solve_device((-q).clone(), z, prof, (480.0, 400.0), [2, 8], **kw)
+    plain = solver.solve_device(q, z, prof, (480.0, 400.0), [2, 8], **kw)
+    assert not torch.equal(want[1], plain[1])
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
