@@ -1,4 +1,6 @@
 #pragma once
+#include <type_traits>
+
 #include "bldfm_passes.h"
 
 // ---------------------------------------------------------------- plain 2-D FFT
@@ -29,25 +31,32 @@ struct StridedOut {
   __device__ __forceinline__ void operator()(int o, double2 v) const { store_as(dst + (int64_t)o * stride, cscale(scale, v)); }
 };
 
-template <int MAXE, class In, class Out>
+// PRIMES: with the butterflies of 7, 11 and 13, for lengths that have such a
+// factor.  They take 109 to 116 registers, the others' kernels 81 to 103; where
+// every length ran them, a small field took longer than it does without:
+// 48 x 64 replayed from a graph 8.5 us against 8.0, 60 x 100 9.5 against 8.3,
+// 512 x 512 14.1 against 13.2.
+inline bool fft2_primes(int n) { return n % 7 == 0 || n % 11 == 0 || n % 13 == 0; }
+
+template <int MAXE, bool PRIMES, class In, class Out>
 __device__ __forceinline__ void fft_plain(bool inv, const FftPlan* F, int n, const double2* __restrict__ tw, int tid,
                                           int T, In in, Out out, bool reuse) {
   const bldfm_fft::Lds buf = bldfm_fft::lds_view(smem, n);
-  if (inv) bldfm_fft::lds_fft<MAXE, true, true>(buf, smem + n, F, tw, tid, T, in, out, reuse);
-  else bldfm_fft::lds_fft<MAXE, false, true>(buf, smem + n, F, tw, tid, T, in, out, reuse);
+  if (inv) bldfm_fft::lds_fft<MAXE, true, PRIMES>(buf, smem + n, F, tw, tid, T, in, out, reuse);
+  else bldfm_fft::lds_fft<MAXE, false, PRIMES>(buf, smem + n, F, tw, tid, T, in, out, reuse);
 }
 
-template <int MAXE, int MAXT, class E>
+template <int MAXE, int MAXT, bool PRIMES, class E>
 __global__ __launch_bounds__(MAXT) void k_fft2_rows(const FftPlan* F, const double2* __restrict__ tw,
                                                   const E* __restrict__ in, double2* __restrict__ mid,
                                                   int32_t n, int64_t nrows, bool inv) {
   const int T = blockDim.x, tid = threadIdx.x;
   for (int64_t r = blockIdx.x; r < nrows; r += gridDim.x)
-    fft_plain<MAXE>(inv, F, n, tw, tid, T, StridedIn<E>{in + r * n, 1}, StridedOut<double2>{mid + r * n, 1, 1.0},
+    fft_plain<MAXE, PRIMES>(inv, F, n, tw, tid, T, StridedIn<E>{in + r * n, 1}, StridedOut<double2>{mid + r * n, 1, 1.0},
                     r != blockIdx.x);
 }
 
-template <int MAXE, int MAXT, class E>
+template <int MAXE, int MAXT, bool PRIMES, class E>
 __global__ __launch_bounds__(MAXT) void k_fft2_cols(const FftPlan* F, const double2* __restrict__ tw,
                                                   const double2* __restrict__ mid, E* __restrict__ out,
                                                   int32_t n0, int32_t n1, int64_t ncols, double scale, bool inv) {
@@ -60,7 +69,7 @@ __global__ __launch_bounds__(MAXT) void k_fft2_cols(const FftPlan* F, const doub
     const int64_t c = gridDim.x >= ncols ? xcd_swizzle(w, ncols) : w;
     const int64_t b = c / n1, col = c % n1;
     const int64_t o = b * (int64_t)n0 * n1 + col;
-    fft_plain<MAXE>(inv, F, n0, tw, tid, T, StridedIn<double2>{mid + o, n1}, StridedOut<E>{out + o, n1, scale},
+    fft_plain<MAXE, PRIMES>(inv, F, n0, tw, tid, T, StridedIn<double2>{mid + o, n1}, StridedOut<E>{out + o, n1, scale},
                     w != blockIdx.x);
   }
 }
@@ -86,7 +95,7 @@ struct TileOut {
     if (live) store_as(dst + (int64_t)o * stride, cscale(scale, v));
   }
 };
-template <int C, class E>
+template <int C, bool PRIMES, class E>
 __global__ __launch_bounds__(1024) void k_fft2_col_tiles(const FftPlan* F, const double2* __restrict__ tw,
                                                        const double2* __restrict__ mid, E* __restrict__ out,
                                                        int32_t n0, int32_t n1, int64_t ntiles, double scale, bool inv) {
@@ -101,8 +110,8 @@ __global__ __launch_bounds__(1024) void k_fft2_col_tiles(const FftPlan* F, const
     const bldfm_fft::LdsT<C> buf = bldfm_fft::lds_view<C>(smem + c, n0);
     const TileIn in{mid + o, n1, live};
     const TileOut<E> dst{out + o, n1, scale, live};
-    if (inv) bldfm_fft::lds_fft<FFT_SMALL_E, true, true>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
-    else bldfm_fft::lds_fft<FFT_SMALL_E, false, true>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
+    if (inv) bldfm_fft::lds_fft<FFT_SMALL_E, true, PRIMES>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
+    else bldfm_fft::lds_fft<FFT_SMALL_E, false, PRIMES>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
   }
 }
 
@@ -170,6 +179,8 @@ int launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, 
   if ((small && threads > 256) || threads > 1024 ||
       (int64_t)threads * (small ? FFT_SMALL_E : BLDFM_FFT_MAXE) < nmax)
     return -1000 - (int)hipErrorInvalidConfiguration;
+  // a one-workgroup pass, its kernel by whether the length has a prime butterfly
+  auto by_primes = [](int n, auto launch) { fft2_primes(n) ? launch(std::true_type()) : launch(std::false_type()); };
   // rows (axis 1, length n1): in -> mid
   if (A1.F1) {
     const unsigned ga = grid_for(nrows * A1.n2, grid_cap), gb = grid_for(nrows * A1.n1, grid_cap);
@@ -182,10 +193,12 @@ int launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, 
       LAUNCH_CHECK();
       k_fft2_long<BLDFM_FFT_MAXE, 1024, true, double2><<<gb, threads, lds_bytes, stream>>>(A1, nullptr, mid, scr, 1, n0, n1, nrows, 1.0, inv);
     }
-  } else if (small) {
-    k_fft2_rows<FFT_SMALL_E, 256, E><<<grid_for(nrows, grid_cap), threads, lds_bytes, stream>>>(A1.F, A1.tw, in, mid, n1, nrows, inv);
   } else {
-    k_fft2_rows<BLDFM_FFT_MAXE, 1024, E><<<grid_for(nrows, grid_cap), threads, lds_bytes, stream>>>(A1.F, A1.tw, in, mid, n1, nrows, inv);
+    by_primes(n1, [&](auto pr) {
+      const unsigned g = grid_for(nrows, grid_cap);
+      if (small) k_fft2_rows<FFT_SMALL_E, 256, pr, E><<<g, threads, lds_bytes, stream>>>(A1.F, A1.tw, in, mid, n1, nrows, inv);
+      else k_fft2_rows<BLDFM_FFT_MAXE, 1024, pr, E><<<g, threads, lds_bytes, stream>>>(A1.F, A1.tw, in, mid, n1, nrows, inv);
+    });
   }
   LAUNCH_CHECK();
   // columns (axis 0, length n0): mid -> out, scaled
@@ -206,24 +219,37 @@ int launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, 
     const int t = (n0 + FFT_SMALL_E - 1) / FFT_SMALL_E;                     // lanes of a column
     const unsigned nt = (unsigned)((t * c + 63) / 64 * 64);
     const size_t lds = ((size_t)n0 * c + tw_table_len(n0)) * 16;
-    if (c == 8) k_fft2_col_tiles<8, E><<<grid_for(tiles, grid_cap), nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
-    else k_fft2_col_tiles<4, E><<<grid_for(tiles, grid_cap), nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
-  } else if (small) {
-    k_fft2_cols<FFT_SMALL_E, 256, E><<<grid_for(ncols, grid_cap), threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
+    by_primes(n0, [&](auto pr) {
+      const unsigned g = grid_for(tiles, grid_cap);
+      if (c == 8) k_fft2_col_tiles<8, pr, E><<<g, nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
+      else k_fft2_col_tiles<4, pr, E><<<g, nt, lds, stream>>>(A0.F, A0.tw, mid, out, n0, n1, tiles, scale, inv);
+    });
   } else {
-    k_fft2_cols<BLDFM_FFT_MAXE, 1024, E><<<grid_for(ncols, grid_cap), threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
+    by_primes(n0, [&](auto pr) {
+      const unsigned g = grid_for(ncols, grid_cap);
+      if (small) k_fft2_cols<FFT_SMALL_E, 256, pr, E><<<g, threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
+      else k_fft2_cols<BLDFM_FFT_MAXE, 1024, pr, E><<<g, threads, lds_bytes, stream>>>(A0.F, A0.tw, mid, out, n0, n1, ncols, scale, inv);
+    });
   }
   LAUNCH_CHECK();
   return 0;
 }
 
+template <bool PRIMES, class E>
+void fft2_lds_attr_of(int bytes) {
+  const void* fns[] = {
+      (const void*)k_fft2_rows<FFT_SMALL_E, 256, PRIMES, E>, (const void*)k_fft2_rows<BLDFM_FFT_MAXE, 1024, PRIMES, E>,
+      (const void*)k_fft2_cols<FFT_SMALL_E, 256, PRIMES, E>, (const void*)k_fft2_cols<BLDFM_FFT_MAXE, 1024, PRIMES, E>,
+      (const void*)k_fft2_col_tiles<4, PRIMES, E>, (const void*)k_fft2_col_tiles<8, PRIMES, E>};
+  for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+}
+
 template <class E>
 void fft2_lds_attr(int bytes) {
   const void* fns[] = {
-      (const void*)k_fft2_rows<FFT_SMALL_E, 256, E>,
       (const void*)k_fft2_long<FFT_SMALL_E, 256, false, E>, (const void*)k_fft2_long<FFT_SMALL_E, 256, true, E>,
-      (const void*)k_fft2_rows<BLDFM_FFT_MAXE, 1024, E>, (const void*)k_fft2_cols<BLDFM_FFT_MAXE, 1024, E>,
-      (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, false, E>, (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, true, E>,
-      (const void*)k_fft2_cols<FFT_SMALL_E, 256, E>, (const void*)k_fft2_col_tiles<4, E>, (const void*)k_fft2_col_tiles<8, E>};
+      (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, false, E>, (const void*)k_fft2_long<BLDFM_FFT_MAXE, 1024, true, E>};
   for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  fft2_lds_attr_of<false, E>(bytes);
+  fft2_lds_attr_of<true, E>(bytes);
 }
