@@ -147,22 +147,6 @@ __global__ __launch_bounds__(MAXT) void k_fft2_long(FftSplit S, const E* __restr
   }
 }
 
-// Columns per workgroup of the column pass: as many as 1024 threads of eight
-// values hold (their buffers are then 128 KB), up to a cache line; 0: a column
-// per workgroup, for columns too long for a tile, for fields of less than 1 MB
-// or 256 columns, whose tiles are fewer than the CUs (200 x 256: 10.2 us against
-// 11.2 in tiles, 256 x 256: 11.2 and 11.1, 1000 x 256: 22.5 and 19.5, 512 x 512:
-// 20.4 and 14.2), and where a prime factor above 13 takes the generic stage,
-// which is arithmetic bound and runs best over many small workgroups
-// (2 x 97 x 300: 32 us against 40 for lanes as few as a tile's).
-inline int fft2_tile(int n0, int64_t ncols) {
-  int m = n0;
-  for (const int p : {2, 3, 5, 7, 11, 13})
-    while (m % p == 0) m /= p;
-  if (n0 > 2048 || ncols < 256 || n0 * ncols < 65536 || m > 1) return 0;
-  return n0 <= 1024 ? 8 : 4;
-}
-
 template <class E>
 int launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, int32_t batch,
                        const E* in, double2* mid, double2* scr, E* out, int32_t sign, double scale,
@@ -213,8 +197,8 @@ int launch_fft2(const FftSplit& A0, int32_t n0, const FftSplit& A1, int32_t n1, 
       LAUNCH_CHECK();
       k_fft2_long<BLDFM_FFT_MAXE, 1024, true, E><<<gb, threads, lds_bytes, stream>>>(A0, nullptr, out, scr, 0, n0, n1, ncols, scale, inv);
     }
-  } else if (fft2_tile(n0, ncols)) {
-    const int c = fft2_tile(n0, ncols);
+  } else if (fft2_tile(n0, n1, batch)) {
+    const int c = fft2_tile(n0, n1, batch);
     const int64_t tiles = (int64_t)batch * ((n1 + c - 1) / c);
     const int t = (n0 + FFT_SMALL_E - 1) / FFT_SMALL_E;                     // lanes of a column
     const unsigned nt = (unsigned)((t * c + 63) / 64 * 64);

@@ -78,6 +78,32 @@ BLDFM_HD int tw_table_len(int n) {
 // Dynamic LDS of one transform: buffer and twiddle tables.
 BLDFM_HD int fft_lds_bytes(int n) { return (n + tw_table_len(n)) * 16; }
 
+// Columns per workgroup of the plain 2-D FFT's column pass: as many as 1024
+// threads of eight values hold (their buffers are then 128 KB), up to a cache
+// line; 0: a column per workgroup.  Both passes in us, a column per workgroup
+// and in tiles:
+//   columns too long for a tile;
+//   fields of less than 1 MB or 256 columns (200 x 256 9.6 and 10.3, 256 x 256 9.8
+//   and 10.0, 512 x 512 13.2 and 13.1, 2 x 2048^2 201 and 131; from 1 to 4 MB columns
+//   of 770 to 1024 points would gain without the tile, 1000 x 256 15.3 and 18.6, and
+//   shorter ones lose, 64 x 64 x 64 28.2 and 26.1);
+//   a prime factor above 13: the generic stage is arithmetic bound and runs best
+//   over many small workgroups (2 x 97 x 300: 30 and 88);
+//   stacks of fields so narrow that most of a tile's lanes have no column (2^21
+//   values, 360 x 1 332 and 400, 360 x 3 297 and 312, 360 x 4 235 and 241, 1024 x 1 588
+//   and 653, 2048 x 3 1017 and 1025; up to 64 points a workgroup is one wave either
+//   way and two live columns pay for the tile: 64 x 1 348 and 351, 16 x 2 493 and 461).
+BLDFM_HD int fft2_tile(int n0, int n1, int64_t batch) {
+  const int64_t ncols = batch * n1;
+  int m = n0;
+  const int smooth[] = {2, 3, 5, 7, 11, 13};
+  for (const int p : smooth)
+    while (m % p == 0) m /= p;
+  if (n0 > 2048 || ncols < 256 || n0 * ncols < 65536 || m > 1) return 0;
+  if (n1 < (n0 > 64 ? 4 : 2)) return 0;
+  return n0 <= 1024 ? 8 : 4;
+}
+
 // Chirp transform of one pass of one instance on a power-of-two length
 // M = 2^lm (bldfm_line.h); lm = 0: the mixed-radix passes run the line.
 struct LineAlg {
