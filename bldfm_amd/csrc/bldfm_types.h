@@ -84,9 +84,9 @@ BLDFM_HD int fft_lds_bytes(int n) { return (n + tw_table_len(n)) * 16; }
 // and in tiles:
 //   columns too long for a tile;
 //   fields of less than 1 MB or 256 columns (200 x 256 9.6 and 10.3, 256 x 256 9.8
-//   and 10.0, 512 x 512 13.2 and 13.1, 2 x 2048^2 201 and 131; from 1 to 4 MB columns
+//   and 10.0, 512 x 512 13.2 and 13.1, 2 x 2048^2 202 and 135; from 1 to 4 MB columns
 //   of 770 to 1024 points would gain without the tile, 1000 x 256 15.3 and 18.6, and
-//   shorter ones lose, 64 x 64 x 64 28.2 and 26.1);
+//   shorter ones lose, 64 x 64 x 64 14.1 and 12.1);
 //   a prime factor above 13: the generic stage is arithmetic bound and runs best
 //   over many small workgroups (2 x 97 x 300: 30 and 88);
 //   stacks of fields so narrow that most of a tile's lanes have no column (2^21
