@@ -125,6 +125,7 @@ SIGNATURES = {
     "bldfm_plan_execute": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P]),
     "bldfm_plan_execute_static": (ctypes.c_int, [_P, _P, _P, _P, _P, _P]),
     "bldfm_plan_timing_begin": (ctypes.c_int, [_P, _I32]),
+    "bldfm_plan_marches": (ctypes.c_int, [_P, ctypes.POINTER(_I32), ctypes.POINTER(_I32)]),
     "bldfm_plan_timing_end": (ctypes.c_int, [_P, ctypes.POINTER(_D), ctypes.POINTER(_I32)]),
     "bldfm_stability": (ctypes.c_int, [_P, _I64, _P, _P, _P]),
     "bldfm_wind_fields": (ctypes.c_int, [_P, _P, _I64, _P, _P, _P]),
@@ -365,6 +366,12 @@ class Plan:
         n = _I32()
         check(load().bldfm_plan_timing_end(self.handle, ms, ctypes.byref(n)), "timing_end")
         return dict(zip(self.PHASES, list(ms))), n.value
+
+    def marches(self):
+        """Instances marched with (one mode, a mode and its mirror) per lane."""
+        one, two = _I32(), _I32()
+        check(load().bldfm_plan_marches(self.handle, ctypes.byref(one), ctypes.byref(two)), "plan_marches")
+        return one.value, two.value
 
     def update_met(self, mets):
         """Replace the meteorology of the plan's instances (a list of Met,

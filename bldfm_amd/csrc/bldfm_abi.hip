@@ -930,6 +930,15 @@ int bldfm_plan_offsets(const bldfm_plan* P, int32_t i, int64_t* off_prof, int64_
   return 0;
 }
 
+int bldfm_plan_marches(const bldfm_plan* P, int32_t* single, int32_t* paired) {
+  if (!P) return fail(BLDFM_EINVAL, "null plan");
+  int32_t n[2] = {0, 0};
+  for (const InstDesc& D : P->desc) ++n[D.pair ? 1 : 0];
+  if (single) *single = n[0];
+  if (paired) *paired = n[1];
+  return 0;
+}
+
 }  // extern "C"
 
 // Workspace of bldfm_plan_execute_static: one array per GPU the library runs

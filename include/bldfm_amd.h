@@ -251,6 +251,13 @@ int bldfm_plan_timing_begin(bldfm_plan* plan, int32_t max_execs);
 int bldfm_plan_timing_end(bldfm_plan* plan, double* phase_ms, int32_t* nexecs);
 
 /*
+ * How the plan marches (no counterpart in the reference; for tests and
+ * benchmarks): the instances marched with one mode per lane, and those with a
+ * mode and its mirror in x per lane.  Results are the same bits either way.
+ */
+int bldfm_plan_marches(const bldfm_plan* plan, int32_t* single, int32_t* paired);
+
+/*
  * 2-D complex FFT of `batch` contiguous (n0, n1) complex128 arrays with
  * numpy semantics: sign -1 (fft2) or +1 (ifft2), every output multiplied by
  * `scale`.  Replaces FFTManager.fft2/ifft2 (src/bldfm/fft_manager.py:78-102).
