@@ -34,7 +34,9 @@ def _level_maps(levels, nz):
     the per-slot level index used by the analytic branch (caller order)."""
     lv = np.asarray(levels)
     slot = np.full(nz, -1, dtype=np.int32)
-    if lv.dtype.kind in "iuf":  # one comparison: ``i in levels`` per level took 1.3 us each
+    # one comparison where it is what ``i in levels`` is (1.3 us a level): not with masked
+    # levels, and not in float16, which rounds i itself
+    if (lv.dtype.kind in "iu" or lv.dtype in (np.float32, np.float64)) and not np.ma.isMaskedArray(levels):
         hit = np.flatnonzero((np.arange(nz)[:, None] == lv.reshape(1, -1)).any(axis=1))
     else:
         hit = [i for i in range(nz) if i in levels]
