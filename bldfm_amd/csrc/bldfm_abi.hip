@@ -169,33 +169,12 @@ void line_tables(const LineAlg& a, double2* out) {
   for (int i = 0; i < M; ++i) put(h[i]);
 }
 
-// How one pass of one instance runs: as a chirp where N has a prime factor
-// above 5 and the chirp's line is the cheaper one.  Both costs are fits of
-// measured passes (us per 1e6 lines, batches of 64^2 to 1000^2 footprints, y-pass):
-// the mixed-radix line of N points takes about N times its stages' sum below,
-// 0.76 p for a prime p > 5 that runs as p products a point, plus 450 (at least
-// 1650: a line is never less than one wave); the chirp takes 1262, 1536, 2836,
-// 7373 and 17760 at M = 128 ... 2048, where from 1024 on a line spans waves.
-// On lengths with factors 2, 3 and 5 alone the chirp is within +-20% of the
-// mixed-radix line up to M = 512 and slower above, so those keep the one
-// transform, whose error is the smaller (conc 3.9-7e-16 against 5-9e-16).
+// How one pass of one instance runs (line_chirp).
 LineAlg choose_line(int N, int nin, int i0, int nout, int o0) {
   LineAlg a;
   memset(&a, 0, sizeof(a));
+  a.lm = line_chirp(N, nin, nout);
   a.N = N; a.nin = nin; a.i0 = i0; a.nout = nout; a.o0 = o0;
-  int lm = LINE_MIN_LM, rest = N;
-  while (lm <= LINE_MAX_LM && nin + nout - 1 > (1 << lm)) ++lm;
-  if (lm > LINE_MAX_LM) return a;
-  double stages = 0.0;
-  for (; rest % 8 == 0; rest /= 8) stages += 0.85;
-  for (; rest % 2 == 0; rest /= 2) stages += 0.4;
-  for (; rest % 3 == 0; rest /= 3) stages += 0.95;
-  for (; rest % 5 == 0; rest /= 5) stages += 1.15;
-  if (rest == 1) return a;
-  for (int p = 7; rest > 1; p += 2)
-    for (; rest % p == 0; rest /= p) stages += 0.76 * p;
-  const double chirp[] = {1250.0, 1262.0, 1536.0, 2836.0, 7373.0, 17760.0};
-  if (chirp[lm - LINE_MIN_LM] < std::max(1650.0, 450.0 + stages * N)) a.lm = lm;
   return a;
 }
 

@@ -117,6 +117,37 @@ struct LineAlg {
 #define LINE_MAX_LM 11
 #define LINE_NLM (LINE_MAX_LM - LINE_MIN_LM + 1)
 
+// log2 of the chirp length that runs a line, or 0 for the mixed-radix line: a
+// chirp where N has a prime factor above 5 and the chirp's line is the cheaper
+// one.  Both costs are fits of measured passes (us per 1e6 lines, mean of y and x,
+// batches of 14^2 to 1008^2 footprints): the mixed-radix line of N points takes
+// about N times its stages' sum below, 1 + 0.64 p for a prime p > 5 that runs as p
+// products a point, plus 600 (at least 1650: a line is never less than one wave).
+// The chirp takes 1262 to 2836 up to M = 512, and from M = 1024 on, where a line
+// spans waves and fewer lines share a CU, 4200 + 4.3 and 13900 + 5 a value of its
+// windows (M = 2048: 19400 at 1084 values, 23700 at 1936).  With one figure a length
+// (7373 and 17760) 704 points of 941 values ran as a chirp in 8470 instead of 7390,
+// 1232 of 1973 in 23550 instead of 20130.  On lengths with factors 2, 3 and 5 alone
+// the chirp is within +-20% of the mixed-radix line up to M = 512 and slower above,
+// so those keep the one transform, whose error is the smaller (conc 3.9-7e-16
+// against 5-9e-16).
+BLDFM_HD int line_chirp(int N, int nin, int nout) {
+  int lm = LINE_MIN_LM, rest = N;
+  while (lm <= LINE_MAX_LM && nin + nout - 1 > (1 << lm)) ++lm;
+  if (lm > LINE_MAX_LM) return 0;
+  double stages = 0.0;
+  for (; rest % 8 == 0; rest /= 8) stages += 0.85;
+  for (; rest % 2 == 0; rest /= 2) stages += 0.4;
+  for (; rest % 3 == 0; rest /= 3) stages += 0.95;
+  for (; rest % 5 == 0; rest /= 5) stages += 1.15;
+  if (rest == 1) return 0;
+  for (int p = 7; rest > 1; p += 2)
+    for (; rest % p == 0; rest /= p) stages += 1.0 + 0.64 * p;
+  const double mixed = 600.0 + stages * N, w = nin + nout;
+  const double chirp = lm == 11 ? 13900.0 + 5.0 * w : lm == 10 ? 4200.0 + 4.3 * w : lm == 9 ? 2836.0 : lm == 8 ? 1536.0 : 1262.0;
+  return chirp < (mixed > 1650.0 ? mixed : 1650.0) ? lm : 0;
+}
+
 // Lines per 256-thread workgroup, stage twiddles in LDS, pitch of the staged
 // lines (the lanes of an LDS access that go to different lines hit different
 // banks) and dynamic LDS of a tile, all for M = 2^lm.
