@@ -294,6 +294,45 @@ __global__ __launch_bounds__(256, 4) void k_line(PlanDev P, ExecBufs B, const Ti
   }
 }
 
+// The tiles of all lengths of one pass in one launch, a workgroup each: length
+// 2^(LINE_MIN_LM + k) has the workgroups first[k] .. first[k + 1] - 1.  A launch a
+// length cost each further length 4 to 5 us of a tail that fills no CU: whole
+// batches of three to seven instances with windows of 28 to 208 values took 68 to 83
+// us, 10 to 17 more than all in the mixed radix, and take 43 to 44.  The switch
+// stands outside any loop: inside the tile loop every length's indices were hoisted
+// out of it (500 registers spilled); so it takes 92 and 108, as the kernels of one
+// length do.
+//
+// Up to LINE_MERGE_TILES: where the tiles fill the chip many times over, all lengths
+// having the longest's LDS (65 KB, two workgroups a CU) costs more than the tails
+// (seven instances of M = 64 .. 2048 each k times, about 950 k tiles a pass, launched
+// apart and together: k = 4 419 and 373 us, 16 1352 and 1342, 24 1995 and 1989, 32 2592
+// and 2673; three of M = 256 .. 1024 each 64 times, 12000 tiles, 675 and 675).
+#define LINE_MERGE_TILES 8192
+struct LineTiles {
+  const TileRec* recs[LINE_NLM];
+  int32_t first[LINE_NLM + 1];
+};
+template <int PASS>
+__global__ __launch_bounds__(256, 4) void k_lines(PlanDev P, ExecBufs B, LineTiles L) {
+  const int b = (int)blockIdx.x;
+  int k = 0;
+  while (b >= L.first[k + 1]) ++k;
+  const TileRec tr = tile_rec(L.recs[k], b - L.first[k]);
+  const cdesc_t& D = *(const cdesc_t*)(P.desc + tr.inst);
+  const int lm = LINE_MIN_LM + k;
+  bldfm_line::fill_twiddles(line_smem, lm, P.tw + D.line[PASS].tw, (int)threadIdx.x);
+  __syncthreads();
+  double2* ex0 = line_smem + line_tw_len(lm);
+  switch (lm) {
+    case 6: line_tile<6, PASS>(P, B, D, tr.inst, tr.local, ex0, line_smem); break;
+    case 7: line_tile<7, PASS>(P, B, D, tr.inst, tr.local, ex0, line_smem); break;
+    case 8: line_tile<8, PASS>(P, B, D, tr.inst, tr.local, ex0, line_smem); break;
+    case 9: line_tile<9, PASS>(P, B, D, tr.inst, tr.local, ex0, line_smem); break;
+    case 10: line_tile<10, PASS>(P, B, D, tr.inst, tr.local, ex0, line_smem); break;
+    default: line_tile<11, PASS>(P, B, D, tr.inst, tr.local, ex0, line_smem); break;
+  }
+}
 // Launches a plan's lines of one pass, or (lds_attr > 0) only allows that much
 // dynamic LDS in the pass's kernels.
 template <int PASS>
@@ -309,6 +348,28 @@ static int launch_lines(const PlanDev& P, const LinePlan& L, const ExecBufs& B, 
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : -(int)e - 1000;
   };
+  int lengths = 0, lds = 0;
+  int64_t tiles = 0;
+  for (int k = 0; k < LINE_NLM; ++k)
+    if (L.tot[PASS][k] > 0) {
+      ++lengths;
+      tiles += L.tot[PASS][k];
+      lds = L.lds[PASS][k] > lds ? L.lds[PASS][k] : lds;
+    }
+  if (lds_attr > 0) {
+    (void)hipFuncSetAttribute((const void*)&k_lines<PASS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_attr);
+  } else if (lengths > 1 && tiles <= LINE_MERGE_TILES) {
+    LineTiles T;
+    for (int k = 0, at = 0; k <= LINE_NLM; ++k) {
+      T.first[k] = at;
+      if (k == LINE_NLM) break;
+      T.recs[k] = L.recs[PASS][k];
+      at += (int)L.tot[PASS][k];
+    }
+    k_lines<PASS><<<(unsigned)tiles, 256, (size_t)lds, stream>>>(P, B, T);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : -(int)e - 1000;
+  }
   int rc = one(&k_line<PASS, 6>, 0);
   if (!rc) rc = one(&k_line<PASS, 7>, 1);
   if (!rc) rc = one(&k_line<PASS, 8>, 2);
