@@ -236,7 +236,7 @@ struct StageK {
 // the workgroup synchronises before the scatter (the stage works in place)
 // and after it (the next stage reads it).  FIRST: Ns = 1 (no twiddles,
 // k = 0, q = j).
-template <int R, int MAXB, bool INV, bool FIRST, class In, class Out>
+template <int R, int MAXB, bool INV, bool FIRST, bool LOOKUP = false, class In, class Out>
 __device__ __forceinline__ void stage_r(In in, Out out, int n, StageK K, TwLds tw,
                                         int tid, int T) {
   constexpr bool to_lds = is_lds<Out>::value;
@@ -261,11 +261,8 @@ __device__ __forceinline__ void stage_r(In in, Out out, int n, StageK K, TwLds t
       }
       if (!FIRST) {
         const int k = j - (int)__umulhi((unsigned)j, K.magic) * K.Ns;
-        if (R > 5 && R != 8) {
-          // W^{r k stride} looked up for every r: twelve repeated products lose
-          // up to 2.8 times the accuracy of the generic stage (a line of 1001
-          // points: relative L2 4.8e-16 against 2.6e-16, of 2197 7.3 against
-          // 2.7), lookups keep it.  r k stride < n, as k < Ns.
+        if (LOOKUP) {
+          // W^{r k stride} looked up for every r (r k stride < n, as k < Ns)
           if (k != 0) {
 #pragma unroll
             for (int r = 1; r < R; ++r) {
@@ -367,7 +364,13 @@ __device__ __forceinline__ void stage_generic(In in, Out out, int n, int R, Stag
 
 // PRIMES: with the butterflies of 7, 11 and 13 (their registers would cost the
 // solver's passes, whose rough lengths run as chirps, a wave a SIMD).
-template <int MAXE, bool INV, bool FIRST, bool PRIMES, class In, class Out>
+// PRIME_LOOKUP: with every twiddle of theirs from the tables, as the generic stage
+// has them.  Up to twelve repeated products (PRIME_POWERS) are 1 to 7% faster but
+// lose up to 2.8 times its accuracy (a line of 1001 points: relative L2 4.8e-16
+// against 2.6e-16 of the generic stage and 2.3e-16 with lookups, of 2197 points 7.3,
+// 2.7 and 2.4), which only a result rounded to single precision hides.
+enum Primes { PRIME_NONE = 0, PRIME_LOOKUP = 1, PRIME_POWERS = 2 };
+template <int MAXE, bool INV, bool FIRST, Primes PRIMES, class In, class Out>
 __device__ __forceinline__ void run_stage(int R, In in, Out out, int n, StageK K, TwLds tw,
                                           int tid, int T) {
   switch (R) {
@@ -377,10 +380,11 @@ __device__ __forceinline__ void run_stage(int R, In in, Out out, int n, StageK K
     case 5: stage_r<5, (MAXE + 4) / 5, INV, FIRST>(in, out, n, K, tw, tid, T); break;
     case 8: stage_r<8, (MAXE + 7) / 8, INV, FIRST>(in, out, n, K, tw, tid, T); break;
     default:
-      if constexpr (PRIMES) {
-        if (R == 7) return stage_r<7, (MAXE + 6) / 7, INV, FIRST>(in, out, n, K, tw, tid, T);
-        if (R == 11) return stage_r<11, (MAXE + 10) / 11, INV, FIRST>(in, out, n, K, tw, tid, T);
-        if (R == 13) return stage_r<13, (MAXE + 12) / 13, INV, FIRST>(in, out, n, K, tw, tid, T);
+      if constexpr (PRIMES != PRIME_NONE) {
+        constexpr bool LK = PRIMES == PRIME_LOOKUP;
+        if (R == 7) return stage_r<7, (MAXE + 6) / 7, INV, FIRST, LK>(in, out, n, K, tw, tid, T);
+        if (R == 11) return stage_r<11, (MAXE + 10) / 11, INV, FIRST, LK>(in, out, n, K, tw, tid, T);
+        if (R == 13) return stage_r<13, (MAXE + 12) / 13, INV, FIRST, LK>(in, out, n, K, tw, tid, T);
       }
       stage_generic<MAXE, INV, FIRST>(in, out, n, R, K, tw, tid, T);
       break;
@@ -400,7 +404,7 @@ __device__ __forceinline__ void run_stage(int R, In in, Out out, int n, StageK K
 // buf synchronises the workgroup before its scatter.
 // tid0, T0: this lane's index and the lanes of its line (the whole workgroup
 // for C = 1); twbuf: the tables' place, behind the C buffers.
-template <int MAXE, bool INV, bool PRIMES = false, int C, class In, class Out>
+template <int MAXE, bool INV, Primes PRIMES = PRIME_NONE, int C, class In, class Out>
 __device__ __forceinline__ void lds_fft(LdsT<C> buf, double2* twbuf, const FftPlan* Pg,
                                         const double2* __restrict__ twg, int tid0, int T0, In in, Out out, bool reuse) {
   typedef const __attribute__((address_space(4))) FftPlan cplan;

@@ -38,7 +38,13 @@ struct StridedOut {
 // 512 x 512 14.1 against 13.2.
 inline bool fft2_primes(int n) { return n % 7 == 0 || n % 11 == 0 || n % 13 == 0; }
 
-template <int MAXE, bool PRIMES, class In, class Out>
+// How they take their twiddles, by the caller's element.
+template <bool PRIMES, class E>
+constexpr bldfm_fft::Primes prime_mode() {
+  return !PRIMES ? bldfm_fft::PRIME_NONE : sizeof(E) == sizeof(double2) ? bldfm_fft::PRIME_LOOKUP : bldfm_fft::PRIME_POWERS;
+}
+
+template <int MAXE, bldfm_fft::Primes PRIMES, class In, class Out>
 __device__ __forceinline__ void fft_plain(bool inv, const FftPlan* F, int n, const double2* __restrict__ tw, int tid,
                                           int T, In in, Out out, bool reuse) {
   const bldfm_fft::Lds buf = bldfm_fft::lds_view(smem, n);
@@ -52,7 +58,7 @@ __global__ __launch_bounds__(MAXT) void k_fft2_rows(const FftPlan* F, const doub
                                                   int32_t n, int64_t nrows, bool inv) {
   const int T = blockDim.x, tid = threadIdx.x;
   for (int64_t r = blockIdx.x; r < nrows; r += gridDim.x)
-    fft_plain<MAXE, PRIMES>(inv, F, n, tw, tid, T, StridedIn<E>{in + r * n, 1}, StridedOut<double2>{mid + r * n, 1, 1.0},
+    fft_plain<MAXE, prime_mode<PRIMES, E>()>(inv, F, n, tw, tid, T, StridedIn<E>{in + r * n, 1}, StridedOut<double2>{mid + r * n, 1, 1.0},
                     r != blockIdx.x);
 }
 
@@ -69,7 +75,7 @@ __global__ __launch_bounds__(MAXT) void k_fft2_cols(const FftPlan* F, const doub
     const int64_t c = gridDim.x >= ncols ? xcd_swizzle(w, ncols) : w;
     const int64_t b = c / n1, col = c % n1;
     const int64_t o = b * (int64_t)n0 * n1 + col;
-    fft_plain<MAXE, PRIMES>(inv, F, n0, tw, tid, T, StridedIn<double2>{mid + o, n1}, StridedOut<E>{out + o, n1, scale},
+    fft_plain<MAXE, prime_mode<PRIMES, E>()>(inv, F, n0, tw, tid, T, StridedIn<double2>{mid + o, n1}, StridedOut<E>{out + o, n1, scale},
                     w != blockIdx.x);
   }
 }
@@ -110,8 +116,8 @@ __global__ __launch_bounds__(1024) void k_fft2_col_tiles(const FftPlan* F, const
     const bldfm_fft::LdsT<C> buf = bldfm_fft::lds_view<C>(smem + c, n0);
     const TileIn in{mid + o, n1, live};
     const TileOut<E> dst{out + o, n1, scale, live};
-    if (inv) bldfm_fft::lds_fft<FFT_SMALL_E, true, PRIMES>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
-    else bldfm_fft::lds_fft<FFT_SMALL_E, false, PRIMES>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
+    if (inv) bldfm_fft::lds_fft<FFT_SMALL_E, true, prime_mode<PRIMES, E>()>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
+    else bldfm_fft::lds_fft<FFT_SMALL_E, false, prime_mode<PRIMES, E>()>(buf, smem + n0 * C, F, tw, t, T, in, dst, w != blockIdx.x);
   }
 }
 
