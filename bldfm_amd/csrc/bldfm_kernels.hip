@@ -287,6 +287,9 @@ __global__ __launch_bounds__(BLOCK, MAXS == 1 ? 5 : 3) void k_shoot(PlanDev P, E
 // so the operations that a pair shares are its gain: 128 footprints of 512^2 x
 // 64 take 1.44e9 vector instructions instead of 1.57e9 and 10% fewer cycles, of
 // which the lower clock (1.83 against 1.99 GHz) takes half: 2.74 -> 2.64 ms.
+// With one snapshot it is at its 128 registers (four waves a SIMD) and spills two
+// to four, stored and reloaded once a tile outside the march: 593 MB of traffic
+// for 539, where the one-mode march has 570.
 template <bool RECOMP, int BLOCK>
 __global__ __launch_bounds__(BLOCK, 4) void k_shoot_pair(PlanDev P, ExecBufs B, int variant) {
   for (int64_t t = blockIdx.x; t < P.tot_shoot; t += gridDim.x) {

@@ -8,7 +8,8 @@
 // 18:451, 1970) that is a convolution of length M >= nin + nout - 1: two
 // transforms of length M and three tables.  What it costs depends on the
 // windows, a third of N each at the default halo, and not on N's factors, where
-// the mixed-radix passes run a prime p > 5 as p products a point.
+// the mixed-radix passes run a prime p > 5 as p products a point.  Windows of more
+// than 2048 values (above 1024 cells an axis at the default halo) stay there.
 //
 // One workgroup of 256 threads takes 2048/M lines; a line's T = M/8 lanes sit
 // in one wave up to M = 512, so its exchanges through LDS need no barrier.  At
@@ -279,8 +280,8 @@ __device__ __forceinline__ void line_tile(const PlanDev& P, const ExecBufs& B, c
   }
 }
 
-// One kernel per pass and length: in one body with a switch over the lengths
-// the compiler kept every length's indices live and spilled 500 registers.
+// One kernel per pass and length: with a switch over the lengths inside this
+// loop the compiler kept every length's indices live and spilled 500 registers.
 template <int PASS, int LM>
 __global__ __launch_bounds__(256, 4) void k_line(PlanDev P, ExecBufs B, const TileRec* recs, int64_t tot) {
   double2* ex0 = line_smem + line_tw_len(LM);

@@ -210,8 +210,8 @@ __device__ __forceinline__ void stage_dyn(const uint8_t* __restrict__ net, SurDy
 // Epilogue of hidden layer l for one wave's accumulators: x = SiLU(z) into the
 // LDS tile (LAST: folded into the two fp32 outputs, per-wave partial sums in
 // red).  FOLD: z is the accumulator itself (the products started from the
-// biases).  TRAIN: also stores z_l and x_{l+1} (bf16) feature-major at point
-// offset p0.
+// biases).  TRAIN: also stores x_{l+1} (bf16, feature-major) and z_l (bf16, in
+// accumulator order) at point offset p0.
 template <bool TRAIN, bool FOLD, bool LAST>
 __device__ __forceinline__ void layer_epilogue(const f32x16 (&acc)[2][4], const SurDyn* dyn, int l, __bf16* act,
                                                float* red, __bf16* __restrict__ xs, __bf16* __restrict__ zs,
