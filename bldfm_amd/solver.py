@@ -144,6 +144,9 @@ def _profiles_to_device(arrays, dev):
         flat = [a if torch.is_tensor(a) else torch.as_tensor(np.asarray(a, dtype=np.float64)) for a in arrays]
         return torch.cat([t.to(device=dev, dtype=torch.float64).reshape(-1) for t in flat])
     flat = [np.asarray(a, dtype=np.float64).reshape(-1) for a in arrays]
+    if torch.cuda.is_current_stream_capturing():
+        # the copy would be recorded, and replays read a block that has other owners by then
+        raise RuntimeError("a solve from host profiles cannot be captured in a graph")
     host = torch.empty(sum(a.size for a in flat), dtype=torch.float64, pin_memory=True)
     np.concatenate(flat, out=host.numpy())
     return host.to(device=dev, non_blocking=True)
