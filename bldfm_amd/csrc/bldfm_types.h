@@ -198,6 +198,10 @@ struct InstDesc {
   int32_t variant;         // shooting kernel: 0 one register snapshot, 1 up to four,
                            // 2 two-pass march, 3 analytic
   int32_t exact;           // 1: reference rounding (no fused multiply-add) in the march
+  int32_t pair, plane;     // 1: marched by k_shoot_pair; its lanes (beside variant and exact, which
+                           // every workgroup of the march reads first: the served batch's march
+                           // takes 0.105 ms, 0.108 with them at the end)
+  int32_t nyq_direct;      // 1: every Nyquist mode's mirror is outside the retained modes
   int32_t snap_level[4];   // level of output slot s < 4 of the numerical branch, or -1
   double dx, dy;
   double sx, sy;        // wavenumber scales ((2 pi)/dx)/nxe, ((2 pi)/dy)/nye
@@ -221,8 +225,6 @@ struct InstDesc {
   int64_t off_long;     // workspace double2: four-step scratch (lines x n of the longest split pass)
   int32_t long_x, long_y;  // 1: the padded x / y length is split (four-step passes)
   LineAlg line[4];         // forward rows, forward columns, inverse y-pass, inverse x-pass
-  int32_t pair, plane;     // 1: marched by k_shoot_pair; its lanes
-  int32_t nyq_direct;      // 1: every Nyquist mode's mirror is outside the retained modes
 };
 
 // ---------------------------------------------------------------- frequencies
